@@ -1505,7 +1505,7 @@ static size_t split_bytes(const GemmArgs& a, int S) {
 // fp32 (every GEMM of the fp32 mode): the matrix cores run fp32 at 1/16 of the bf16 rate, so
 // operand traffic is minor and the tile choice only has to fill the CUs: a round of resident
 // tiles runs per_cu tiles per CU side by side, so its cost is per_cu x the tile's area.
-static BfCfg pick_f32(const GemmArgs& a) {
+[[maybe_unused]] static BfCfg pick_f32(const GemmArgs& a) {
   if (a.N <= 32 && !a.qk_dim) return CFG_128x32;
   if (a.N <= 64 && !a.qk_dim) return CFG_F64x64;
   const BfCfg cands[] = {CFG_256x256, CFG_256x128, CFG_F128x128, CFG_F64x64};
@@ -1521,16 +1521,17 @@ static BfCfg pick_f32(const GemmArgs& a) {
   return pick;
 }
 
+template <typename T>
 static bool launch_f32_auto(const Exec& ex, const GemmArgs& a) {
   const BfCfg c = pick_f32(a);
   int S = split_factor(a, c);
   if (S > 1 && !(ex.ws && ex.ws->ptr && ex.ws->cap >= split_bytes(a, S))) S = 1;
   switch (c) {
-    case CFG_128x32: return launch_mfma<float, 128, 32, 4, 1, 2>(ex, a, S);
-    case CFG_256x256: return launch_mfma<float, 256, 256, 2, 4, 2>(ex, a, S);
-    case CFG_256x128: return launch_mfma<float, 256, 128, 4, 2, 3>(ex, a, S);
-    case CFG_F128x128: return launch_mfma<float, 128, 128, 2, 2, 2>(ex, a, S);
-    default: return launch_mfma<float, 64, 64, 2, 2, 2>(ex, a, S);
+    case CFG_128x32: return launch_mfma<T, 128, 32, 4, 1, 2>(ex, a, S);
+    case CFG_256x256: return launch_mfma<T, 256, 256, 2, 4, 2>(ex, a, S);
+    case CFG_256x128: return launch_mfma<T, 256, 128, 4, 2, 3>(ex, a, S);
+    case CFG_F128x128: return launch_mfma<T, 128, 128, 2, 2, 2>(ex, a, S);
+    default: return launch_mfma<T, 64, 64, 2, 2, 2>(ex, a, S);
   }
 }
 
@@ -1742,7 +1743,7 @@ __global__ void __launch_bounds__(576, 1) conv3x3_halo_kernel(const GemmArgs p, 
 // Which convolutions take conv3x3_halo_kernel: 3x3, stride 1, padding 1, Cin and Cout 32 or 64,
 // plain row stores without LayerScale, 16-byte aligned epilogue operands, and rows of at least
 // 64 pixels (narrower maps waste most of a 32-column tile).
-static bool conv_halo_ok(const GemmArgs& a) {
+[[maybe_unused]] static bool conv_halo_ok(const GemmArgs& a) {
   return a.amode == A_CONV && a.ks == 3 && a.stride == 1 && a.pad == 1 && a.Ho == a.Hi && a.Wo == a.Wi &&
          (a.Cin == 32 || a.Cin == 64) && (a.N == 32 || a.N == 64) && a.store == STORE_ROWS && !a.rm_P && !a.hw3 &&
          !a.ln_in && !a.ln_out && !a.qk_dim && !a.glu && !a.q_cols && !a.gamma && a.epi_vec && a.Wo >= 64 &&
@@ -1821,11 +1822,15 @@ static bool mfma_path_ok(const GemmArgs& a) {
   return abytes < 2147483648.0 && double(a.N) * a.ldw * es < 2147483648.0;
 }
 
+// The kernels of one operand type. This file is compiled once per type (SPLAT_GEMM_TYPE = float,
+// bf16 or f16: the instantiations below) and once without it (gemm() itself), side by side.
+template <typename T> bool launch_typed(const Exec& ex, const GemmArgs& a);
+#ifdef SPLAT_GEMM_TYPE
 template <typename T>
-static bool launch_typed(const Exec& ex, const GemmArgs& a) {
+bool launch_typed(const Exec& ex, const GemmArgs& a) {
   if (mfma_path_ok(a)) {
     if constexpr (sizeof(T) == 2) return launch_h16_auto<T>(ex, a);
-    else return launch_f32_auto(ex, a);
+    else return launch_f32_auto<T>(ex, a);
   }
   SPLAT_CHECK(a.hw3 == nullptr && a.ln_in == nullptr, BAD_ARGUMENT,
               "gemm: the fused head and the folded LayerNorm need the MFMA path");
@@ -1836,6 +1841,9 @@ static bool launch_typed(const Exec& ex, const GemmArgs& a) {
   else launch_cfg<T, 64, 128, 1, 4>(ex, a);
   return false;
 }
+
+template bool launch_typed<SPLAT_GEMM_TYPE>(const Exec& ex, const GemmArgs& a);
+#else
 
 void gemm(const Exec& ex, const GemmArgs& args) {
   GemmArgs a = args;
@@ -1892,5 +1900,6 @@ void gemm(const Exec& ex, const GemmArgs& args) {
   if (a.ln_out && !stats)  // this path's epilogue does not emit them
     ln_stats(ex, static_cast<const float*>(a.out), a.ldc, a.M, a.N, a.ln_group, a.ln_out, a.dt, a.ln_copy);
 }
+#endif
 
 }  // namespace splat
