@@ -7,13 +7,11 @@
 // first 16 bytes of a 32-byte k-step, lanes 32-63 the second; A and W use the same k order,
 // so the sum over k is exact whatever order the hardware walks the fragment in.
 //   bf16: one v_mfma_f32_32x32x16_bf16 per k-step;
-//   fp32: 64-byte k-steps on v_mfma_f32_16x16x4_f32 (it sustains ~145 TFLOP/s on this part,
-//   v_mfma_f32_32x32x2_f32 ~120): lane l reads 16 bytes of row l%16 of each 16-row half of a
-//   32-row tile, chunk 4 s + l/16 of the step, and product e of a half pair takes float e of
-//   those fragments (k-slot l/16 = chunk l/16).
-// Accumulator layout per 32x32 tile (f32x16): bf16, lane l, register r -> row 8*(r/4) +
-// 4*(l/32) + r%4, column l%32; fp32, registers 4 (2 mi + ni) + r -> row 16 mi + 4*(l/16) + r,
-// column 16 ni + l%16.
+//   fp32: 64-byte k-steps (two 16-byte chunks a lane); every float is split exactly into three
+//   bf16 (split8) and six v_mfma_f32_32x32x16_bf16 sum the products down to 2^-18 of the leading
+//   one (Mfma<float>).
+// Accumulator layout per 32x32 tile (f32x16): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4,
+// column l%32.
 #include "kernels.h"
 
 #include <algorithm>
@@ -52,26 +50,15 @@ template <> struct Mfma<f16> {
   __device__ static inline uint4 relu(uint4 v) { return Mfma<bf16>::relu(v); }  // same sign-bit rule
 };
 template <> struct Mfma<float> {
-  // One 64-byte k-step of a 32x32 tile as 2 x 2 halves of 16 rows / 16 columns: a0, a1 the A
-  // fragments of rows 0-15 and 16-31, b0, b1 the W fragments of columns 0-15 and 16-31.
-  __device__ static inline void mma2x2(f32x16& acc, const uint4& a0, const uint4& a1, const uint4& b0,
-                                       const uint4& b1) {
-    f32x4 c0 = acc.s0123, c1 = acc.s4567, c2 = acc.s89ab, c3 = acc.scdef;
-    const float* x0 = reinterpret_cast<const float*>(&a0);
-    const float* x1 = reinterpret_cast<const float*>(&a1);
-    const float* y0 = reinterpret_cast<const float*>(&b0);
-    const float* y1 = reinterpret_cast<const float*>(&b1);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x0[e], y0[e], c0, 0, 0, 0);
-      c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x0[e], y1[e], c1, 0, 0, 0);
-      c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[e], y0[e], c2, 0, 0, 0);
-      c3 = __builtin_amdgcn_mfma_f32_16x16x4f32(x1[e], y1[e], c3, 0, 0, 0);
-    }
-    acc.s0123 = c0;
-    acc.s4567 = c1;
-    acc.s89ab = c2;
-    acc.scdef = c3;
+  // a . b without the terms below 2^-26 of the leading one (m l, l m, l l): the five small
+  // products into `low`, the leading one into `acc` (they may be one accumulator).
+  __device__ static inline void mma_split(f32x16& acc, f32x16& low, const Split8& a, const Split8& b) {
+    Mfma<bf16>::mma(low, a.m, b.m);
+    Mfma<bf16>::mma(low, a.h, b.l);
+    Mfma<bf16>::mma(low, a.l, b.h);
+    Mfma<bf16>::mma(low, a.h, b.m);
+    Mfma<bf16>::mma(low, a.m, b.h);
+    Mfma<bf16>::mma(acc, a.h, b.h);
   }
   __device__ static inline void mma(f32x16& acc, const uint4& a, const uint4& b) {
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
@@ -252,23 +239,14 @@ template <> struct LdsFloats<0> {
 };
 
 
-template <int TM, int TN, bool L16>
+template <int TM, int TN>
 __device__ __forceinline__ void stage_slab(const f32x16 (&acc)[TM][TN], int i, float* slab, int lane) {
   constexpr int LD = slab_ld(TN);
-  if constexpr (L16) {  // fp32: 16x16 halves, registers 4 (2 mi + ni) + r
-    const int q = lane >> 4, l16 = lane & 15;
+  const int g = lane >> 5, l32 = lane & 31;
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+  for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        slab[(16 * (r >> 3) + 4 * q + (r & 3)) * LD + j * 32 + 16 * ((r >> 2) & 1) + l16] = acc[i][j][r];
-  } else {
-    const int g = lane >> 5, l32 = lane & 31;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) slab[(8 * (r >> 2) + 4 * g + (r & 3)) * LD + j * 32 + l32] = acc[i][j][r];
-  }
+    for (int r = 0; r < 16; ++r) slab[(8 * (r >> 2) + 4 * g + (r & 3)) * LD + j * 32 + l32] = acc[i][j][r];
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -376,7 +354,7 @@ __device__ inline void qk_norm_rope(const GemmArgs& p, float (&v)[CH][8], const 
 // `lnab` (EPI_LN): (rstd, -rstd * mean) of this wave's rows in LDS; `xch` (EPI_LN with
 // qk_dim): the block's qk-norm exchange area, xrow0 this wave's first tile row. `lnp`
 // (EPI_RESLN): this wave's corner of the LDS array of 32-column sums, lnp_ld a row.
-template <typename T, int TM, int TN, int EPI, bool L16 = false>
+template <typename T, int TM, int TN, int EPI>
 __device__ __forceinline__ void epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN], long wrow0, long wcol0, float* slab,
                                          int lane, bool vec, float* part = nullptr, const float* lnab = nullptr,
                                          float* lnp = nullptr, int lnp_ld = 0, float* xch = nullptr, int xrow0 = 0) {
@@ -385,7 +363,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN
     // rows of 8 columns: n < N implies n + 8 <= ldp (ldp is N rounded up to 8)
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      stage_slab<TM, TN, L16>(acc, i, slab, lane);
+      stage_slab(acc, i, slab, lane);
       for (int q = lane; q < 32 * RUNS; q += 64) {
         const int rr = q / RUNS, cc = (q - rr * RUNS) * 8;
         const long m = wrow0 + i * 32 + rr, n = wcol0 + cc;
@@ -400,7 +378,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN
   } else if constexpr (EPI == EPI_FULL) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      stage_slab<TM, TN, L16>(acc, i, slab, lane);
+      stage_slab(acc, i, slab, lane);
       for (int q = lane; q < 32 * RUNS; q += 64) {
         const int rr = q / RUNS, cc = (q - rr * RUNS) * 8;
         const long m = wrow0 + i * 32 + rr, n = wcol0 + cc;
@@ -459,7 +437,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN
           lb[t] = ab.y;
         }
       }
-      stage_slab<TM, TN, L16>(acc, i, slab, lane);
+      stage_slab(acc, i, slab, lane);
 #pragma unroll
       for (int t0 = 0; t0 < IT; t0 += CH) {
         float v[CH][8], rv[CH][8];
@@ -585,7 +563,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN
 // lane takes 8 channels of a slab row: h = bf16(relu(acc + bias)), 6 partial dot products with
 // the 1x1 weights, summed over the row's lanes by DPP; the waves' partials per row meet in LDS
 // after the slabs (the ring is free by then), and one thread per pixel finishes the outputs.
-template <typename T, int BM, int BN, int WM, int WN, int TM, int TN, bool L16 = false>
+template <typename T, int BM, int BN, int WM, int WN, int TM, int TN>
 __device__ __forceinline__ void head_epilogue(const GemmArgs& p, f32x16 (&acc)[TM][TN], long m0, int wm, int wn,
                                               float* smemf, int wave, int lane, int tid) {
   constexpr int NW = WM * WN, COLS = TN * 32, LD = slab_ld(TN), RUNS = COLS / 8, RPP = 64 / RUNS;
@@ -603,7 +581,7 @@ __device__ __forceinline__ void head_epilogue(const GemmArgs& p, f32x16 (&acc)[T
   for (int k = 0; k < 8; ++k) cb[k] = p.bias[c0 + k];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    stage_slab<TM, TN, L16>(acc, i, slab, lane);
+    stage_slab(acc, i, slab, lane);
 #pragma unroll
     for (int t = 0; t < 32 / RPP; ++t) {
       const int rr = rsub + t * RPP;
@@ -853,9 +831,62 @@ constexpr uint32_t OOB = 0x80000000u;
 // at most 32 taps (chosen by the launcher; callers pass A_CONV): each k-tile lies in one tap.
 constexpr int A_CONV_TAP = 2;
 
-// T = bf16 (one v_mfma_f32_32x32x16_bf16 per k-step) or float (four v_mfma_f32_32x32x2f32):
-// a k-step is 32 bytes of K per row either way, so the tiles, loads and swizzles are the same
-// byte for byte; BK counts elements (128-byte rows: 64 bf16 or 32 fp32).
+// An fp32 wave whose sums are not all finite takes them again from the operands as they are, on
+// v_mfma_f32_32x32x2_f32: split8 turns an infinity (and a value that rounds to one in bf16) into
+// NaN, which must not reach outputs that are infinite or finite. Rows of A or W past the operand
+// are zeros, as in the main loop. Rare, so it reads global memory without staging.
+template <int TM, int TN, bool CONV, bool RELU>
+__device__ inline void plain_products(const GemmArgs& p, f32x16 (&acc)[TM][TN], long wrow0, long wcol0, int k0, int k1,
+                                      int lane) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t = fmaf(acc[i][j][r], 0.f, t);  // NaN once a sum is not finite
+  if (!__any(t != 0.f)) return;
+  const int g = lane >> 5, l32 = lane & 31;
+  const float* A = reinterpret_cast<const float*>(p.A);
+  const float* W = reinterpret_cast<const float*>(p.W);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  for (int k = k0 + g; k < k1; k += 2) {  // k0 and k1 are even
+    float a[TM], b[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const long m = wrow0 + i * 32 + l32;
+      a[i] = 0.f;
+      if (m >= p.M) continue;
+      if constexpr (CONV) {
+        const int hw = p.Ho * p.Wo, v = int(m / hw), rem = int(m - long(v) * hw);
+        const int tap = k / p.Cin, ci = k - tap * p.Cin;
+        const int iy = rem / p.Wo * p.stride - p.pad + tap / p.ks, ix = rem % p.Wo * p.stride - p.pad + tap % p.ks;
+        if (iy >= 0 && iy < p.Hi && ix >= 0 && ix < p.Wi) a[i] = A[((long(v) * p.Hi + iy) * p.Wi + ix) * p.Cin + ci];
+      } else {
+        a[i] = A[m * p.lda + k];
+      }
+      if (RELU) a[i] = __int_as_float(max(__float_as_int(a[i]), 0));
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const long n = wcol0 + j * 32 + l32;
+      b[j] = n < p.N ? W[n * p.ldw + k] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+}
+
+// T = bf16 (one v_mfma_f32_32x32x16_bf16 per 32-byte k-step) or float (six of them per 64-byte
+// k-step): the tiles, loads and swizzles are the same byte for byte; BK counts elements (128-byte
+// rows: 64 bf16 or 32 fp32).
 // MINB: blocks per CU the register allocation must allow (2 for a tile whose LDS ring lets two
 // blocks share a CU).
 // AR: ring stages of the A tiles (STAGES those of W). AR = 3 with two W stages (the 256x256 tile,
@@ -866,17 +897,23 @@ template <typename T, int BM, int BN, int WM, int WN, int STAGES, int BK, int AM
 __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const GemmArgs p, int tiles_m, int tiles_n) {
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32, NW = WM * WN;
   constexpr int ES = sizeof(T), KE = 16 / ES;  // bytes per element, elements per 16-byte chunk
-  constexpr int MPI = ES == 4 ? 16 : 1;        // MFMA instructions per tile pair and k-step
+  constexpr int MPI = ES == 4 ? 6 : 1;         // MFMA instructions per tile pair and k-step
   // A tile row holds BK elements = RB bytes = CPR 16-byte chunks; one load instruction of a
   // wave fills RPI rows (1 KiB). Chunk c of row r sits in slot c ^ ((r >> SH) & (CPR - 1)), which
   // keeps the 16 lanes of every ds_read_b128 phase on distinct banks.
   constexpr int RB = BK * ES, CPR = RB / 16, RPI = 64 / CPR, SH = CPR == 8 ? 1 : 2;
   static_assert(RB == 128 || RB == 64, "k-tile");
-  // fp32: 64-byte k-steps on 16x16x4 products, two fragments (16-row halves) per 32-row tile
-  constexpr bool L16 = ES == 4;
-  static_assert(!L16 || RB == 128, "fp32 k-tiles are 128 bytes");
-  constexpr int KS = L16 ? RB / 64 : RB / 32;
-  constexpr int FH = L16 ? 2 : 1;  // fragments per 32-row tile per k-step
+  // fp32: 64-byte k-steps, two 16-byte chunks per 32-row tile and lane, split into bf16 parts
+  constexpr bool F32T = ES == 4;
+  static_assert(!F32T || RB == 128, "fp32 k-tiles are 128 bytes");
+  // fp32: the small products get accumulators of their own, so that the large sum is rounded once a
+  // k-step and not six times, where the registers allow it (a 64x64 wave tile would lose its
+  // second block a CU: 5838x384x1536 58 -> 67 us). Error against 64 bits (2-norm over the
+  // result's) at K = 384 / 1536 / 2048: 0.8 / 1.7 / 2.0e-7, without 2.1 / 4.3 / 5.0e-7; on the fp32
+  // instructions 2.5 / 5.0 / 5.8e-7.
+  constexpr bool LOW = F32T && TM * TN < 4;
+  constexpr int KS = F32T ? RB / 64 : RB / 32;
+  constexpr int FH = F32T ? 2 : 1;  // 16-byte fragments per 32-row tile per k-step
   constexpr int AL = BM / (NW * RPI), BL = BN / (NW * RPI);  // load instructions per wave per k-tile
   constexpr int LPT = AL + BL;
   static_assert(AL * NW * RPI == BM && BL * NW * RPI == BN, "tile rows split evenly over the waves' loads");
@@ -1032,12 +1069,10 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  // fragment rows are frow plus multiples of 32 (bf16: l32) or 16 (fp32: l%16)
-  const int frow = L16 ? (lane & 15) : l32, fsub = L16 ? (lane >> 4) : g;
-  const int sw = (frow >> SH) & (CPR - 1);
-  const int arow0 = (wm * (BM / WM) + frow) * RB, brow0 = (BM + wn * (BN / WN) + frow) * RB;
-  // byte offset of this lane's chunk in k-step s of a tile row
-  auto step_off = [&](int st) { return (((L16 ? 4 : 2) * st + fsub) ^ sw) * 16; };
+  const int sw = (l32 >> SH) & (CPR - 1);
+  const int arow0 = (wm * (BM / WM) + l32) * RB, brow0 = (BM + wn * (BN / WN) + l32) * RB;
+  // byte offset of this lane's chunk h in k-step s of a tile row
+  auto step_off = [&](int st, int h) { return (((FH * st + h) * 2 + g) ^ sw) * 16; };
   // Prologue: AHEAD tiles in flight, tile 0 resident for every wave, its first fragments read.
   // Every k-tile slot is loaded, also past the last tile (as zeros), so that the number of
   // loads in flight, and with it each vmcnt wait, is the same for every tile.
@@ -1046,7 +1081,7 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
   // up the wave that issues it, so loads crowded into one step leave the matrix core idle (the
   // 6222x1024x4096 GEMM on 256x128 tiles: 61 -> 52 us). With two stages a stage frees only at
   // the barrier, and the loads of tile kt + 2 go into the barrier step.
-  constexpr bool SPREAD = STAGES >= 3;
+  constexpr bool SPREAD = STAGES >= 3 && !F32T;
   constexpr int AHEAD = SPREAD ? STAGES - 1 : STAGES;  // tile kt loads tile kt + AHEAD
   // Folded LayerNorm: thread r < BM loads the partial statistics of tile row r ahead of the
   // operand tiles (up to 16 pairs) and reduces them once the first stage is resident.
@@ -1099,109 +1134,180 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
   uint4 fa[2][TM * FH], fb[2][TN * FH];
   // Fragment f of a k-step in the order the MFMAs (i outer, j inner) first use them: the A
   // fragments of tile row 0, then every W fragment, then the other A ones, so that the first
-  // MFMAs of a step wait for few reads. Fragment rows are 32 / FH apart.
+  // MFMAs of a step wait for few reads. Fragment f: chunk f % FH of 32-row tile f / FH.
   // k-tile kt's A rows at abase(kt) + arow0.., its W rows at wbase(kt) + brow0.. (brow0 counts
   // the BM A rows of a whole stage)
   auto abase = [&](int kt) -> const char* { return smem + (SPLITR ? (kt % AR) * BM * RB : (kt % STAGES) * STAGE); };
   auto wbase = [&](int kt) -> const char* {
     return SPLITR ? smem + AR * BM * RB + (kt % STAGES) * BN * RB - BM * RB : smem + (kt % STAGES) * STAGE;
   };
-  auto read_frag = [&](int kt, int off, int slot, int f) {
-    constexpr int RS = 32 / FH * RB;
+  auto read_frag = [&](int kt, int st, int slot, int f) {
+    constexpr int RS = 32 * RB;
+    const int off = step_off(st, f % FH);
     const char* sa = abase(kt);
     const char* sw_ = wbase(kt);
-    if (f < FH) fa[slot][f] = *reinterpret_cast<const uint4*>(sa + arow0 + f * RS + off);
-    else if (f < FH + TN * FH) fb[slot][f - FH] = *reinterpret_cast<const uint4*>(sw_ + brow0 + (f - FH) * RS + off);
-    else fa[slot][f - TN * FH] = *reinterpret_cast<const uint4*>(sa + arow0 + (f - TN * FH) * RS + off);
+    if (f < FH) fa[slot][f] = *reinterpret_cast<const uint4*>(sa + arow0 + off);
+    else if (f < FH + TN * FH) fb[slot][f - FH] = *reinterpret_cast<const uint4*>(sw_ + brow0 + (f - FH) / FH * RS + off);
+    else fa[slot][f - TN * FH] = *reinterpret_cast<const uint4*>(sa + arow0 + (f - TN * FH) / FH * RS + off);
   };
   auto read_frags = [&](int kt, int s, int slot) {
-    const int off = step_off(s);
 #pragma unroll
-    for (int f = 0; f < (TM + TN) * FH; ++f) read_frag(kt, off, slot, f);
+    for (int f = 0; f < (TM + TN) * FH; ++f) read_frag(kt, s, slot, f);
   };
   // the products of tile pair (i, j) for the k-step whose fragments sit in `slot`
-  auto mma = [&](int i, int j, int slot) {
-    if constexpr (L16)
-      Mfma<float>::mma2x2(acc[i][j], fa[slot][2 * i], fa[slot][2 * i + 1], fb[slot][2 * j], fb[slot][2 * j + 1]);
-    else
-      Mfma<T>::mma(acc[i][j], fa[slot][i], fb[slot][j]);
-  };
-  read_frags(0, 0, 0);
-  // One k-tile; the last one is peeled (HAS_NEXT false) so that each step's reads and MFMAs
-  // share a basic block and the LDS waits stay exact.
-  constexpr int MM = TM * TN, NF = (TM + TN) * FH, CUR = (KS - 1) & 1;
-  auto tile = [&](int kt, auto has_next, auto full) {
-    constexpr bool HAS_NEXT = decltype(has_next)::value;
+  auto mma = [&](int i, int j, int slot) { Mfma<T>::mma(acc[i][j], fa[slot][i], fb[slot][j]); };
+  if constexpr (F32T) {
+    // The matrix cores work on the parts of one k-step while the VALU splits the next step's
+    // fragments and the LDS reads of the one after are in flight: a wave on its own would run the
+    // three one after the other. Tile kt is read from LDS during tile kt - 1, so at the barrier that
+    // opens tile kt (tile kt + 1 resident) its stage is free for tile kt + STAGES.
+    Split8 pa[2][TM], pb[2][TN];
+    f32x16 low[LOW ? TM : 1][LOW ? TN : 1];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      // hard fence: the reads below belong to this step's region and nothing moves across
-      __builtin_amdgcn_sched_barrier(0);
-      if (RELU) {
+    for (int i = 0; i < (LOW ? TM : 1); ++i)
 #pragma unroll
-        for (int i = 0; i < TM * FH; ++i) fa[s & 1][i] = Mfma<T>::relu(fa[s & 1][i]);
+      for (int j = 0; j < (LOW ? TN : 1); ++j) low[i][j] = f32x16{};
+    constexpr int MM = TM * TN, NF = (TM + TN) * FH, NS = TM + TN;
+    constexpr int SV = (NS * 44 / MM + 5) / 6;  // VALU instructions of the splits after each MFMA
+    // fragments of `slot` -> parts of the same k-step parity
+    auto split_frag = [&](int slot, int f) {
+      if (f < TN) {
+        pb[slot][f] = split8(fb[slot][2 * f], fb[slot][2 * f + 1]);
+      } else {
+        uint4 x = fa[slot][2 * (f - TN)], y = fa[slot][2 * (f - TN) + 1];
+        if (RELU) {
+          x = Mfma<float>::relu(x);
+          y = Mfma<float>::relu(y);
+        }
+        pa[slot][f - TN] = split8(x, y);
       }
-      if ((SPREAD || (SPLITR && HAS_NEXT)) && s + 1 < KS) {
-        // this step's share of the loads of tile kt + AHEAD (split ring: of the A rows of tile
-        // kt + 2 only) and the reads of the next step's fragments, spread between the MFMAs
-        constexpr int LS = SPLITR ? AL : LPT;
-        const int L0 = s * LS / (KS - 1), L1 = (s + 1) * LS / (KS - 1);
-        const int off = step_off(s + 1);
+    };
+    read_frags(0, 0, 0);
+    read_frags(0, 1, 1);
+#pragma unroll
+    for (int f = 0; f < NS; ++f) split_frag(0, f);
+    auto tile = [&](int kt, auto has_next, auto full) {
+      constexpr bool HAS_NEXT = decltype(has_next)::value;
+      if constexpr (HAS_NEXT) {
+        wait_vmcnt<(STAGES - 2) * LPT>();
+        __syncthreads();
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        // product q of the step with its share of the splits, the reads and (step 0) the loads
 #pragma unroll
         for (int q = 0; q < MM; ++q) {
-          mma(q / TN, q % TN, s & 1);
-#pragma unroll
-          for (int l = L0 + q * (L1 - L0) / MM; l < L0 + (q + 1) * (L1 - L0) / MM; ++l)
-            issue_one(kt + AHEAD, (kt + AHEAD) % STAGES, l, full);
-#pragma unroll
-          for (int r = q * NF / MM; r < (q + 1) * NF / MM; ++r) read_frag(kt, off, (s + 1) & 1, r);
           __builtin_amdgcn_sched_barrier(0);
-        }
-      } else if (s + 1 < KS || !HAS_NEXT) {
-        if (s + 1 < KS) read_frags(kt, s + 1, (s + 1) & 1);
+          if constexpr (HAS_NEXT) {
+            if (s == 0) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+              for (int l = q * LPT / MM; l < (q + 1) * LPT / MM; ++l) issue_one(kt + STAGES, kt % STAGES, l, full);
+            }
 #pragma unroll
-          for (int j = 0; j < TN; ++j) mma(i, j, s & 1);
-        if (s + 1 < KS) {
-          // interleave the LDS reads with this step's MFMAs
+            for (int r = q * NF / MM; r < (q + 1) * NF / MM; ++r) read_frag(kt + 1, s, s, r);
+          }
+          if (HAS_NEXT || s == 0) {
 #pragma unroll
-          for (int k = 0; k < NF; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, MM * MPI / NF > 0 ? MM * MPI / NF : 1, 0);
+            for (int f = q * NS / MM; f < (q + 1) * NS / MM; ++f) split_frag(s ^ 1, f);
+          }
+          f32x16& c = acc[q / TN][q % TN];
+          Mfma<float>::mma_split(c, LOW ? low[LOW ? q / TN : 0][LOW ? q % TN : 0] : c, pa[s][q / TN], pb[s][q % TN]);
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, SV, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
           }
         }
-      } else {
-        // Last step of a tile with a successor. Every wave holds its last fragments of tile kt
-        // (the barrier waits for LDS reads), so the stage of tile kt is free once tile kt+1 is
-        // resident (tiles kt+2 .. kt+STAGES-1 may still be in flight). With two stages the
-        // loads of tile kt+2 and the reads of the next tile's first fragments are spread
-        // between this step's MFMAs, in a fixed order; with more, only the reads.
-        // Split ring: tile kt+1 is resident once at most the AL loads of A tile kt+2 are in
-        // flight; then the W loads of tile kt+2 go out.
-        wait_vmcnt<SPLITR ? AL : (STAGES - 2) * LPT>();
-        __syncthreads();
-        const int off0 = step_off(0);
-        constexpr int LB = SPLITR ? AL : 0, LN_ = LPT - LB;
-#pragma unroll
-        for (int q = 0; q < MM; ++q) {
-          mma(q / TN, q % TN, CUR);
-          if constexpr (!SPREAD) {
-#pragma unroll
-            for (int l = LB + q * LN_ / MM; l < LB + (q + 1) * LN_ / MM; ++l) issue_one(kt + STAGES, kt % STAGES, l, full);
-          }
-#pragma unroll
-          for (int r = q * NF / MM; r < (q + 1) * NF / MM; ++r) read_frag(kt + 1, off0, 0, r);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    };
+    int kt = 0;
+    for (; kt + 1 < nk && kt + STAGES < nk_full; ++kt) tile(kt, std::true_type{}, std::true_type{});
+    for (; kt + 1 < nk; ++kt) tile(kt, std::true_type{}, std::false_type{});
+    tile(nk - 1, std::false_type{}, std::false_type{});
+    if constexpr (LOW) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
     }
-  };
-  // tiles whose loads are of a full tile (kt + AHEAD), then the rest; the last is peeled
-  int kt = 0;
-  for (; kt + 1 < nk && kt + AHEAD < nk_full; ++kt) tile(kt, std::true_type{}, std::true_type{});
-  for (; kt + 1 < nk; ++kt) tile(kt, std::true_type{}, std::false_type{});
-  tile(nk - 1, std::false_type{}, std::false_type{});
+  } else {
+    read_frags(0, 0, 0);
+    // One k-tile; the last one is peeled (HAS_NEXT false) so that each step's reads and MFMAs
+    // share a basic block and the LDS waits stay exact.
+    constexpr int MM = TM * TN, NF = (TM + TN) * FH, CUR = (KS - 1) & 1;
+    auto tile = [&](int kt, auto has_next, auto full) {
+      constexpr bool HAS_NEXT = decltype(has_next)::value;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        // hard fence: the reads below belong to this step's region and nothing moves across
+        __builtin_amdgcn_sched_barrier(0);
+        if (RELU) {
+#pragma unroll
+          for (int i = 0; i < TM * FH; ++i) fa[s & 1][i] = Mfma<T>::relu(fa[s & 1][i]);
+        }
+        if ((SPREAD || (SPLITR && HAS_NEXT)) && s + 1 < KS) {
+          // this step's share of the loads of tile kt + AHEAD (split ring: of the A rows of tile
+          // kt + 2 only) and the reads of the next step's fragments, spread between the MFMAs
+          constexpr int LS = SPLITR ? AL : LPT;
+          const int L0 = s * LS / (KS - 1), L1 = (s + 1) * LS / (KS - 1);
+#pragma unroll
+          for (int q = 0; q < MM; ++q) {
+            mma(q / TN, q % TN, s & 1);
+#pragma unroll
+            for (int l = L0 + q * (L1 - L0) / MM; l < L0 + (q + 1) * (L1 - L0) / MM; ++l)
+              issue_one(kt + AHEAD, (kt + AHEAD) % STAGES, l, full);
+#pragma unroll
+            for (int r = q * NF / MM; r < (q + 1) * NF / MM; ++r) read_frag(kt, s + 1, (s + 1) & 1, r);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else if (s + 1 < KS || !HAS_NEXT) {
+          if (s + 1 < KS) read_frags(kt, s + 1, (s + 1) & 1);
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) mma(i, j, s & 1);
+          if (s + 1 < KS) {
+            // interleave the LDS reads with this step's MFMAs
+#pragma unroll
+            for (int k = 0; k < NF; ++k) {
+              __builtin_amdgcn_sched_group_barrier(0x008, MM * MPI / NF > 0 ? MM * MPI / NF : 1, 0);
+              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+          }
+        } else {
+          // Last step of a tile with a successor. Every wave holds its last fragments of tile kt
+          // (the barrier waits for LDS reads), so the stage of tile kt is free once tile kt+1 is
+          // resident (tiles kt+2 .. kt+STAGES-1 may still be in flight). With two stages the
+          // loads of tile kt+2 and the reads of the next tile's first fragments are spread
+          // between this step's MFMAs, in a fixed order; with more, only the reads.
+          // Split ring: tile kt+1 is resident once at most the AL loads of A tile kt+2 are in
+          // flight; then the W loads of tile kt+2 go out.
+          wait_vmcnt<SPLITR ? AL : (STAGES - 2) * LPT>();
+          __syncthreads();
+          constexpr int LB = SPLITR ? AL : 0, LN_ = LPT - LB;
+#pragma unroll
+          for (int q = 0; q < MM; ++q) {
+            mma(q / TN, q % TN, CUR);
+            if constexpr (!SPREAD) {
+#pragma unroll
+              for (int l = LB + q * LN_ / MM; l < LB + (q + 1) * LN_ / MM; ++l) issue_one(kt + STAGES, kt % STAGES, l, full);
+            }
+#pragma unroll
+            for (int r = q * NF / MM; r < (q + 1) * NF / MM; ++r) read_frag(kt + 1, 0, 0, r);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // tiles whose loads are of a full tile (kt + AHEAD), then the rest; the last is peeled
+    int kt = 0;
+    for (; kt + 1 < nk && kt + AHEAD < nk_full; ++kt) tile(kt, std::true_type{}, std::true_type{});
+    for (; kt + 1 < nk; ++kt) tile(kt, std::true_type{}, std::false_type{});
+    tile(nk - 1, std::false_type{}, std::false_type{});
+  }
   wait_vmcnt<0>();  // the zero-fill loads past the last tile must land before the ring is reused
   __syncthreads();  // every wave is past its last read of the ring before slabs reuse it
   if constexpr (SPLITR && EPI == EPI_LN) {
@@ -1211,15 +1317,18 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
     }
     __syncthreads();
   }
-  if constexpr (sizeof(T) == 4) __builtin_amdgcn_s_setprio(0);
+  if constexpr (F32T) {
+    __builtin_amdgcn_s_setprio(0);
+    plain_products<TM, TN, AMODE != A_ROWS, RELU>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kt0 * BK, kend, lane);
+  }
   if constexpr (EPI == EPI_HEAD) {
     static_assert(NW * 32 * slab_ld(TN) * 4 + BM * WN * 6 * 4 <= RING, "head epilogue LDS");
-    head_epilogue<T, BM, BN, WM, WN, TM, TN, L16>(p, acc, m0, wm, wn, reinterpret_cast<float*>(smem), wave, lane, tid);
+    head_epilogue<T, BM, BN, WM, WN, TM, TN>(p, acc, m0, wm, wn, reinterpret_cast<float*>(smem), wave, lane, tid);
   } else {
     float* slab = reinterpret_cast<float*>(smem) + wave * 32 * slab_ld(TN);
     constexpr int LNLD = BN / 32;  // 32-column sums per tile row (EPI_RESLN)
     float* lnp = reinterpret_cast<float*>(smem) + NW * 32 * slab_ld(TN);
-    epilogue<T, TM, TN, EPI, L16>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), slab, lane, p.epi_vec,
+    epilogue<T, TM, TN, EPI>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), slab, lane, p.epi_vec,
                              EPI == EPI_PART ? p.part + long(split) * p.M * p.ldp : nullptr,
                              EPI == EPI_LN ? lnab + wm * (BM / WM) * 2 : nullptr,
                              lnp + (wm * (BM / WM) * LNLD + wn * (BN / WN) / 32) * 2, LNLD,
@@ -1300,7 +1409,7 @@ constexpr int GEMM_CUS = 256;  // MI355X compute units: one "round" of resident 
 // order in time matters more than the union of panels (8192^3, four rounds: contiguous runs
 // 1.30 PFLOP/s, the round-robin deal 1.01), so those keep the default.
 struct XcdTileMap { int tm, tn, bm, bn, group, contig; };
-static void xcd_tile_map(GemmArgs& b, int tm, int tn, int bm, int bn) {
+[[maybe_unused]] static void xcd_tile_map(GemmArgs& b, int tm, int tn, int bm, int bn) {
   const int nblk = tm * tn;
   if (nblk > 2 * GEMM_CUS) return;
   static thread_local std::vector<XcdTileMap> cache;
@@ -1421,7 +1530,7 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
 
 // Tile configurations of the bf16 path: block tile, and how many blocks share a CU.
 enum BfCfg { CFG_128x32, CFG_128x64, CFG_256x256, CFG_256x128, CFG_320x256, CFG_320x128, CFG_192x128, CFG_128x128,
-             CFG_F128x128, CFG_F64x64, CFG_192x128D };
+             CFG_F128x128, CFG_F64x64, CFG_192x128D, CFG_F128x64 };
 struct BfShape { int bm, bn, per_cu; };
 static BfShape bf_shape(BfCfg c) {
   switch (c) {
@@ -1435,6 +1544,7 @@ static BfShape bf_shape(BfCfg c) {
     case CFG_F128x128: return {128, 128, 2};
     case CFG_F64x64: return {64, 64, 4};
     case CFG_192x128D: return {192, 128, 2};
+    case CFG_F128x64: return {128, 64, 3};
     default: return {128, 128, 1};
   }
 }
@@ -1449,7 +1559,7 @@ static BfShape bf_shape(BfCfg c) {
 // tiles (QKV 6222x3072x1024: 59.5 us as 600 tiles of 256x128, 48.5 as 480 of 320x128, 42.3);
 // 192x128 (8 waves of 96x32, 3 stages) puts N = 768 in one round of 198 smaller tiles
 // (6223x768x3072 42.4 -> 38.4 us).
-static BfCfg pick_bf16(const GemmArgs& a) {
+[[maybe_unused]] static BfCfg pick_bf16(const GemmArgs& a) {
   // Narrow outputs (the DA3 head's 32/64-channel convs): 128-row tiles and two stages keep the
   // LDS per block at 40-48 KB, so 3-4 blocks share a CU and hide each other's load latency
   // (C2 convs 475 -> 266 us against 256-row tiles with 3-4 stages).
@@ -1487,14 +1597,24 @@ static BfCfg pick_bf16(const GemmArgs& a) {
 // spans at least 16 k-tiles is cut into S >= 2 slices of at least 8 k-tiles, S * tiles within
 // one round. The slices write fp32 partials; a second kernel sums them and applies the
 // epilogue (the DPT head's coarse-level convs: M = 1596, K = 6912, 14 tiles of 256x128).
+// fp32 (64x64 tiles): at most 160 tiles, one round of slices of at least 6 k-tiles or two rounds of at
+// least 12 (us unsplit / split, the reduce included: 1297x384x1536 126 tiles 31.6 / 22.4 in 4; 3x3 of 64
+// channels, K = 576: 81 tiles 16.8 / 14.2 in 3, 21 tiles 16.2 / 12.1 in 3; 324 tiles lose, 26.2 / 29.7).
 static int split_factor(const GemmArgs& a, BfCfg c) {
   if (a.hw3 || a.ln_in) return 1;  // the fused head needs whole tiles, a folded LayerNorm whole rows of K
   const BfShape sh = bf_shape(c);
   const long tiles = long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn);
   const long slots = long(GEMM_CUS) * sh.per_cu;
   const int nk = cdiv(a.K, a.dt == F32 ? 32 : 64);
-  if (2 * tiles > slots || nk < 16) return 1;
-  const int S = int(std::min<long>(nk / 8, slots / tiles));
+  int S;
+  if (c == CFG_F64x64) {
+    if (tiles > 160) return 1;
+    S = int(std::max(std::min<long>(nk / 6, GEMM_CUS / tiles), std::min<long>(nk / 12, 2 * GEMM_CUS / tiles)));
+    S = std::min(S, 16);
+  } else {
+    if (2 * tiles > slots || nk < 16) return 1;
+    S = int(std::min<long>(nk / 8, slots / tiles));
+  }
   if (S < 2) return 1;
   return cdiv(nk, cdiv(nk, S));  // every slice non-empty
 }
@@ -1502,21 +1622,27 @@ static size_t split_bytes(const GemmArgs& a, int S) {
   return S > 1 ? size_t(S) * a.M * ((a.N + 7) / 8 * 8) * sizeof(float) : 0;
 }
 
-// fp32 (every GEMM of the fp32 mode): the matrix cores run fp32 at 1/16 of the bf16 rate, so
-// operand traffic is minor and the tile choice only has to fill the CUs: a round of resident
-// tiles runs per_cu tiles per CU side by side, so its cost is per_cu x the tile's area.
+// fp32: six matrix products of split parts a k-step, and 44 VALU instructions for every 8 values
+// a wave splits, so a wave's share of the tile sets the ratio of the two: 64x64 (128x128 tiles)
+// is bound by the matrix cores, 32x32 (64x64 tiles) by the VALU. Cost of a choice: the tiles of
+// the fullest CU times area / eff, and a wave alone on its SIMD overlaps less except in the 64x64
+// shape. Measured (bias epilogue, us for 128x128 / 128x64 / 64x64): 5838x1152x384 37 / 45 / 50,
+// 5838x384x1536 58 / 74 / 72, 1297x1152x384 20 / 16 / 17, 1297x384x384 18 / 14 / 10, 8192x2048x2048
+// 354 / 432 / 506; 3x3 of 64 channels on 93312 pixels 56 on 128x64, 65 on 64x64.
+// A launch that 64x64 tiles would leave under half full and K allows keeps them and splits K.
 [[maybe_unused]] static BfCfg pick_f32(const GemmArgs& a) {
   if (a.N <= 32 && !a.qk_dim) return CFG_128x32;
-  if (a.N <= 64 && !a.qk_dim) return CFG_F64x64;
-  const BfCfg cands[] = {CFG_256x256, CFG_256x128, CFG_F128x128, CFG_F64x64};
+  if (split_factor(a, CFG_F64x64) > 1) return CFG_F64x64;
+  const BfCfg cands[] = {CFG_F128x128, CFG_F128x64, CFG_F64x64};
+  const double eff[] = {1.0, 0.82, 0.69}, alone[] = {1.0, 1.15, 1.15};
   double best = 1e30;
-  BfCfg pick = CFG_256x256;
-  for (BfCfg c : cands) {
-    const BfShape sh = bf_shape(c);
-    const long tiles = long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn);
-    const long slots = long(GEMM_CUS) * sh.per_cu;
-    const double cost = double((tiles + slots - 1) / slots) * sh.per_cu * sh.bm * sh.bn;
-    if (cost < best * 0.999) { best = cost; pick = c; }
+  BfCfg pick = CFG_F128x128;
+  for (int i = 0; i < 3; ++i) {
+    const BfShape sh = bf_shape(cands[i]);
+    if (a.N <= 64 && sh.bn > 64) continue;
+    const long per = (long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn) + GEMM_CUS - 1) / GEMM_CUS;
+    const double cost = double(per) * sh.bm * sh.bn / eff[i] * (per == 1 ? alone[i] : 1.0);
+    if (cost < best * 0.999) { best = cost; pick = cands[i]; }
   }
   return pick;
 }
@@ -1528,9 +1654,8 @@ static bool launch_f32_auto(const Exec& ex, const GemmArgs& a) {
   if (S > 1 && !(ex.ws && ex.ws->ptr && ex.ws->cap >= split_bytes(a, S))) S = 1;
   switch (c) {
     case CFG_128x32: return launch_mfma<T, 128, 32, 4, 1, 2>(ex, a, S);
-    case CFG_256x256: return launch_mfma<T, 256, 256, 2, 4, 2>(ex, a, S);
-    case CFG_256x128: return launch_mfma<T, 256, 128, 4, 2, 3>(ex, a, S);
     case CFG_F128x128: return launch_mfma<T, 128, 128, 2, 2, 2>(ex, a, S);
+    case CFG_F128x64: return launch_mfma<T, 128, 64, 2, 2, 2>(ex, a, S);
     default: return launch_mfma<T, 64, 64, 2, 2, 2>(ex, a, S);
   }
 }

@@ -1,0 +1,114 @@
+"""fp32 products from three bf16 parts (gemm, convolutions) against float64: sizes at the
+edges of the tiles, wide ranges, and operands that are infinite, NaN or round to infinity in bf16.
+
+Tolerance (2-norm of the error over the result's): the parts are exact and the products left out are
+below 3 * 2^-26; what is left are the roundings of the sum, at most six for every 16 values of K, each
+below 2^-24 of the sum and independent: 2^-24 sqrt(6 K / 16).
+"""
+import numpy as np
+import pytest
+
+from conftest import report
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+import splathip
+
+
+def _tol(K):
+    return 2.0 ** -24 * (6 * max(K, 16) / 16) ** 0.5 + 3 * 2.0 ** -26
+
+
+def _rand(g, *shape):
+    return torch.randn(*shape, generator=g).cuda()
+
+
+def _gemm(ctx, A, W, bias):
+    M, K = A.shape
+    N = W.shape[0]
+    ldw = (K + 63) // 64 * 64
+    Wp = torch.zeros(N, ldw, device="cuda")
+    Wp[:, :K] = W
+    out = torch.full((M, N), -7.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_gemm(splathip.F32, A.data_ptr(), M, K, Wp.data_ptr(), N, ldw, bias.data_ptr(), 0, out.data_ptr(), True)
+    ctx.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 4), (31, 32, 32), (33, 24, 68), (64, 64, 96), (65, 72, 36),        # 128x32 and 64x64 tiles, K tails
+    (1297, 384, 384), (1297, 1152, 384), (200, 64, 1536), (65, 64, 3456),     # 64x64, 128x64; K split
+    (2100, 1152, 64), (5838, 384, 100), (4097, 512, 128),                     # 128x128, ragged last tiles
+])
+def test_gemm_matches_float64(ctx, M, N, K):
+    g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
+    A, W, b = _rand(g, M, K), _rand(g, N, K) * K ** -0.5, _rand(g, N)
+    out = _gemm(ctx, A, W, b).double()
+    ref = A.double() @ W.double().t() + b.double()
+    err = float((out - ref).norm() / ref.norm())
+    report("f32.gemm", M=M, N=N, K=K, err=f"{err:.2e}", tol=f"{_tol(K):.2e}")
+    assert err <= _tol(K)
+
+
+@pytest.mark.parametrize("exp", [-55, 40])
+def test_gemm_wide_range(ctx, exp):
+    """Rows and columns spread over 2^+-20 around 2^exp: every row is right by itself."""
+    g = torch.Generator().manual_seed(5)
+    A = _rand(g, 130, 256) * torch.exp2(torch.randint(-20, 21, (130, 1), generator=g).float() + exp).cuda()
+    W = _rand(g, 96, 256) * torch.exp2(torch.randint(-20, 21, (96, 1), generator=g).float()).cuda()
+    out = _gemm(ctx, A, W, torch.zeros(96, device="cuda")).double()
+    ref = A.double() @ W.double().t()
+    scale = A.double().norm(dim=1)[:, None] * W.double().norm(dim=1)[None]
+    err = float(((out - ref) / scale).norm() / (ref / scale).norm())
+    assert err <= _tol(256)
+
+
+def _same(out, ref, tol):
+    """NaN, infinities and their signs in the same places; the rest within tol."""
+    out, ref = out.double(), ref.double()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
+    fine = torch.isfinite(ref)
+    assert torch.isfinite(out[fine]).all()
+    err = float((out[fine] - ref[fine]).norm() / ref[fine].norm())
+    assert err <= tol, err
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 96, 64), (140, 64, 1536), (2100, 1152, 64)])  # 64x64 / 128x64, split, 128x128
+def test_gemm_special_values(ctx, M, N, K):
+    g = torch.Generator().manual_seed(9)
+    A, W = _rand(g, M, K), _rand(g, N, K)
+    A[3, 5], A[40, 7], A[41, K - 1] = float("inf"), float("nan"), float("-inf")
+    W[9, 2] = float("inf")
+    A[50] = 0.0
+    A[50, 1], W[:, 1] = 3.4e38, W[:, 1].clamp(-0.5, 0.5)   # rounds to infinity in bf16, the product is finite
+    W[9, 1] = 0.25
+    out = _gemm(ctx, A, W, torch.zeros(N, device="cuda"))
+    ref = A.double().cpu() @ W.double().cpu().t()
+    rows = [r for r in range(M) if r != 50]
+    _same(out.cpu()[rows], ref[rows], _tol(K))
+    keep = [c for c in range(N) if c != 9]
+    _same(out.cpu()[50, keep], ref[50, keep].float(), 1e-6)
+
+
+@pytest.mark.parametrize("V,H,W,C,N,relu", [(1, 5, 7, 64, 64, 1), (2, 18, 18, 96, 64, 0), (1, 70, 66, 32, 32, 0),
+                                            (1, 40, 33, 48, 40, 0), (3, 108, 144, 64, 64, 1)])
+def test_conv_matches_float64(ctx, V, H, W, C, N, relu):
+    g = torch.Generator().manual_seed(H * W + C)
+    x, w, b = _rand(g, V, H, W, C), _rand(g, N, C, 3, 3) * (9 * C) ** -0.5, _rand(g, N)
+    ldw = (9 * C + 63) // 64 * 64
+    wp = torch.zeros(N, ldw, device="cuda")
+    wp[:, :9 * C] = w.permute(0, 2, 3, 1).reshape(N, -1)
+    out = torch.empty(V, H, W, N, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_conv2d(splathip.F32, x.data_ptr(), V, H, W, C, wp.data_ptr(), N, ldw, 3, 1, b.data_ptr(), relu, 0, 0,
+                      out.data_ptr())
+    ctx.synchronize()
+    xin = (x.clamp(min=0) if relu else x).cpu().double().permute(0, 3, 1, 2)
+    ref = torch.nn.functional.conv2d(xin, w.cpu().double(), b.cpu().double(), padding=1).permute(0, 2, 3, 1)
+    err = float((out.cpu().double() - ref).norm() / ref.norm())
+    report("f32.conv", V=V, H=H, W=W, C=C, N=N, err=f"{err:.2e}")
+    assert err <= _tol(9 * C)
