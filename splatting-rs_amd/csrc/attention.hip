@@ -747,19 +747,26 @@ __global__ void __launch_bounds__(WAVES * 64, QT == 1 ? 4 : 2) attn_bf16_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// fp32 path. 4 waves x 32 queries, 32-key tiles. K and V tiles stream straight into LDS (rows of
-// 256 bytes = 64 fp32 head channels, 16-byte chunk c of tile row r in slot c ^ (r & 15)), two
-// ring slots each. S^T = K Q^T on v_mfma_f32_32x32x2f32: k-step j pairs head channels j and
-// j + 32 (lane half g supplies channel j + 32 g), so a lane reads its key row in 16-byte chunks
-// and holds its query's 32 Q values (times log2(e)/8) in registers. The scores' accumulator
-// layout (lane l, register r: key 8 (r/4) + 4 g + r%4, query l%32) is the B operand of
-// O^T = V^T P^T as it stands: product r takes key 8 (r/4) + 4 g + r%4 in its k-slot g, and the
-// A operand reads that key's V row (head channels dt*32 + l%32) with one ds_read_b32. Softmax:
-// the max-free plain pass and the running-max safe pass of the bf16 kernel, P in fp32.
+// fp32 path. 4 waves x 32 queries, 32-key tiles. The plain pass (max-free, as in the bf16 kernel)
+// runs S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16: every operand is split exactly
+// into three bf16 parts (split8) and the six products down to 2^-18 of the leading one are
+// summed, which keeps fp32's precision at 6/16 of the fp32 instructions' matrix time. Q is split
+// once. The block splits each K and V tile once for its four waves: a thread loads 8 channels of
+// one key two tiles ahead, splits them and writes the parts to LDS (three planes of 128-byte
+// rows, laid out as the bf16 kernel's tiles: K chunk c of row r in slot c ^ ((r >> 1) & 7), V in
+// c ^ (2 (r & 3)) for the transposing reads), one tile ahead of its use: two buffers, one barrier a
+// tile. The scores' accumulator layout (lane l, register r: key 8 (r/4) + 4 g + r%4, query l%32)
+// is, split, the B operand of O^T = V^T P^T as it stands.
+// The safe pass (running maximum) keeps the operands whole on v_mfma_f32_32x32x2f32, K and V
+// tiles streamed into LDS (rows of 256 bytes, 16-byte chunk c of row r in slot c ^ (r & 15)): k-step j
+// pairs head channels j and j + 32. It also takes the blocks whose plain pass met an infinity, a
+// NaN, or a value that rounds to infinity in bf16.
 template <bool SPLIT>
 __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, float c) {
-  constexpr int TB = 32 * 256;  // one 32-key K or V tile
-  __shared__ __attribute__((aligned(1024))) char smem[4 * TB];  // K slots 0, 1 then V slots 0, 1
+  constexpr int TB = 32 * 256;            // one 32-key fp32 K or V tile (safe pass)
+  constexpr int PB = 32 * 128, KVB = 6 * PB;  // one plane; K and V planes h, m, l of a tile
+  __shared__ __attribute__((aligned(1024))) char smem[2 * KVB];  // safe pass: K slots 0, 1, V slots 0, 1
+  static_assert(2 * KVB >= 4 * TB, "the safe pass's ring");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
   const int L = p.L;
@@ -770,74 +777,209 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
   const long base = long(sq) * p.seq_stride;
   const int q0 = (qb * 4 + wave) * 32;
   const bool active = __builtin_amdgcn_readfirstlane(q0) < L;
+  const int ntiles = (L + 31) / 32;
+  const int t0 = SPLIT ? split * p.tps : 0, t1 = SPLIT ? min(ntiles, t0 + p.tps) : ntiles;
 
-  float qf[32];  // Q[query q0 + l32][channels 32 g + (0..31)] * c
-  {
-    const int qrow = q0 + l32;
-    const float* Q = reinterpret_cast<const float*>(p.q) + (base + qrow) * p.ld + h * 64 + 32 * g;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float4 v = qrow < L ? *reinterpret_cast<const float4*>(Q + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
-      qf[4 * i] = v.x * c;
-      qf[4 * i + 1] = v.y * c;
-      qf[4 * i + 2] = v.z * c;
-      qf[4 * i + 3] = v.w * c;
-    }
-  }
-
-  // DMA: load instruction i (0, 1) of wave w fills tile rows 16 i + 4 w + lane/16; lane slot
-  // lane%16 holds chunk (lane%16) ^ (row & 15) of that row.
+  // this lane's query row (clamped; zeros past L), times c in fp32 in either pass
+  const bool qok = q0 + l32 < L;
+  const float* Q = reinterpret_cast<const float*>(p.q) + (base + min(q0 + l32, L - 1)) * p.ld + h * 64;
+  auto load_q = [&](int ch) {
+    const float4 v = *reinterpret_cast<const float4*>(Q + ch);
+    return qok ? make_float4(v.x * c, v.y * c, v.z * c, v.w * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
   const float* Kseq = reinterpret_cast<const float*>(p.k) + base * p.ld + h * 64;
   const float* Vseq = reinterpret_cast<const float*>(p.v) + base * p.ld + h * 64;
-  const int32x4_t rk = make_rsrc_a(Kseq, uint32_t(long(L) * p.ld * 4));
-  const int32x4_t rv = make_rsrc_a(Vseq, uint32_t(long(L) * p.ld * 4));
-  int lrw[2];
-  uint32_t goff[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    lrw[i] = 16 * i + 4 * wave + (lane >> 4);
-    goff[i] = uint32_t(lrw[i] * p.ld * 4 + (((lane & 15) ^ (lrw[i] & 15)) * 16));
-  }
-  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((lds_cptr_a)smem));
-  const uint32_t tile_bytes = uint32_t(32 * p.ld * 4);
-  auto issue = [&](int t, auto bufc) {
-    constexpr int B = decltype(bufc)::value;
-    const uint32_t so = uint32_t(t) * tile_bytes;
-    const bool full = t * 32 + 32 <= L;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t vo = (full || t * 32 + lrw[i] < L) ? goff[i] : 0x80000000u;
-      load_lds_a(rk, vo, so, lds0 + B * TB + (16 * i + 4 * wave) * 256);
-      load_lds_a(rv, vo, so, lds0 + (2 + B) * TB + (16 * i + 4 * wave) * 256);
-    }
-  };
 
   f32x16 o[2];
-  float mref, lsum;
-  const int ks = l32 & 15;  // row swizzle of this lane's K row (row l32)
+  float mref = 0.f, lsum = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) { o[0][r] = 0.f; o[1][r] = 0.f; }
+  // keys past L in the last tile weigh nothing
+  auto mask = [&](f32x16& s, int t) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (t * 32 + 8 * (r >> 2) + 4 * g + (r & 3) >= L) s[r] = -INFINITY;
+  };
 
-  auto tile = [&](int t, auto bufc, auto masked_t, auto safe_t) {
-    constexpr bool masked = decltype(masked_t)::value, safe = decltype(safe_t)::value;
-    constexpr int B = decltype(bufc)::value;
-    const char* kb = smem + B * TB;
-    const char* vb = smem + (2 + B) * TB;
-    f32x16 s = {};
-    __builtin_amdgcn_s_setprio(1);  // matrix-core sections first among the SIMD's waves (as above)
+  // ---- plain pass
+  {
+    // a . b of split operands, the small terms first (those below 2^-26 are left out)
+    auto mma_split = [](f32x16& acc, const Split8& x, const Split8& y) {
+      acc = mma16<bf16>(x.m, y.m, acc);
+      acc = mma16<bf16>(x.h, y.l, acc);
+      acc = mma16<bf16>(x.l, y.h, acc);
+      acc = mma16<bf16>(x.h, y.m, acc);
+      acc = mma16<bf16>(x.m, y.h, acc);
+      acc = mma16<bf16>(x.h, y.h, acc);
+    };
+    Split8 q[4];  // channels 16 st + 8 g + (0..7)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {  // channels 4 i .. 4 i + 3 (+ 32 g)
-      const float4 kf = *reinterpret_cast<const float4*>(kb + l32 * 256 + (((8 * g + i) ^ ks) * 16));
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.x, qf[4 * i], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.y, qf[4 * i + 1], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.z, qf[4 * i + 2], s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.w, qf[4 * i + 3], s, 0, 0, 0);
+    for (int st = 0; st < 4; ++st) {
+      const float4 a = load_q(16 * st + 8 * g), b = load_q(16 * st + 8 * g + 4);
+      const float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      q[st] = split8(w);
     }
-    __builtin_amdgcn_s_setprio(0);
-    if constexpr (masked) {
+    // this thread's part of a tile: key row tid / 8, channels 8 (tid % 8) + (0..7)
+    const int trow = tid >> 3, tch = tid & 7;
+    const int kdst = trow * 128 + ((tch ^ ((trow >> 1) & 7)) * 16), vdst = trow * 128 + ((tch ^ (2 * (trow & 3))) * 16);
+    uint4 rk[2], rv[2];
+    // buffer loads: rows at or past L read as zeros
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    const int span = int((long(L - 1) * p.ld + 64) * 4);
+    const auto bk = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Kseq), 0, span, 0x00020000);
+    const auto bv = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Vseq), 0, span, 0x00020000);
+    auto load = [&](int t) {
+      const int key = t * 32 + trow;
+      const int vo = key < L ? int(uint32_t(key) * uint32_t(p.ld * 4) + tch * 32) : int(0x80000000u);
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (t * 32 + 8 * (r >> 2) + 4 * g + (r & 3) >= L) s[r] = -INFINITY;
+      for (int i = 0; i < 2; ++i) {
+        rk[i] = __builtin_bit_cast(uint4, u32x4(__builtin_amdgcn_raw_buffer_load_b128(bk, vo, 16 * i, 0)));
+        rv[i] = __builtin_bit_cast(uint4, u32x4(__builtin_amdgcn_raw_buffer_load_b128(bv, vo, 16 * i, 0)));
+      }
+    };
+    auto store = [&](int buf) {
+      char* kb = smem + buf * KVB;
+      const Split8 k = split8(rk[0], rk[1]), v = split8(rv[0], rv[1]);
+      *reinterpret_cast<uint4*>(kb + kdst) = k.h;
+      *reinterpret_cast<uint4*>(kb + PB + kdst) = k.m;
+      *reinterpret_cast<uint4*>(kb + 2 * PB + kdst) = k.l;
+      *reinterpret_cast<uint4*>(kb + 3 * PB + vdst) = v.h;
+      *reinterpret_cast<uint4*>(kb + 4 * PB + vdst) = v.m;
+      *reinterpret_cast<uint4*>(kb + 5 * PB + vdst) = v.l;
+    };
+    // A operand of the V^T product: vbase[dt] and ds_read_b64_tr_b16 as in the bf16 kernel
+    int vbase[2];
+    {
+      const int G = lane >> 4, vj = (lane >> 2) & 3, vcc = lane & 3;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+        vbase[dt] = (4 * (G >> 1) + vj) * 128 + (((4 * dt + 2 * (G & 1) + (vcc >> 1)) ^ (vj << 1)) * 16) + (vcc & 1) * 8;
     }
-    if constexpr (safe) {
+    auto vfrag = [&](const char* vt, int hh, int dt) {
+      typedef short v4s __attribute__((ext_vector_type(4)));
+      uint32_t w[4];
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) v4s*)((lds_cptr_a)(vt + (16 * hh + 8 * half) * 128 + vbase[dt])));
+        const uint2 u = __builtin_bit_cast(uint2, r);
+        w[2 * half] = u.x;
+        w[2 * half + 1] = u.y;
+      }
+      return make_uint4(w[0], w[1], w[2], w[3]);
+    };
+    const int sw = (l32 >> 1) & 7;
+    auto tile = [&](int t, int buf, auto masked_t) {
+      const char* kb = smem + buf * KVB;
+      const char* vt = kb + 3 * PB;
+      f32x16 s = {};
+      __builtin_amdgcn_s_setprio(1);  // matrix-core sections first among the SIMD's waves (as above)
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const char* kr = kb + l32 * 128 + ((2 * st + g) ^ sw) * 16;
+        const Split8 k = {*reinterpret_cast<const uint4*>(kr), *reinterpret_cast<const uint4*>(kr + PB),
+                          *reinterpret_cast<const uint4*>(kr + 2 * PB)};
+        mma_split(s, k, q[st]);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      if constexpr (decltype(masked_t)::value) mask(s, t);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lsum += s[r];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = s[8 * hh + e];
+        const Split8 ps = split8(w);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) {
+          const Split8 v = {vfrag(vt, hh, dt), vfrag(vt + PB, hh, dt), vfrag(vt + 2 * PB, hh, dt)};
+          mma_split(o[dt], v, ps);
+        }
+        __builtin_amdgcn_s_setprio(0);
+      }
+    };
+    load(t0);
+    store(0);
+    load(t0 + 1);  // rows past L read as zeros, also a whole tile of them
+    for (int t = t0; t < t1; ++t) {
+      const int buf = (t - t0) & 1;
+      __syncthreads();  // tile t is in LDS; every wave is past tile t - 1
+      if (t + 1 < t1) {
+        store(buf ^ 1);
+        load(t + 2);
+      }
+      if (active) {
+        if (t + 1 < t1) tile(t, buf, std::false_type{});
+        else tile(t, buf, std::true_type{});  // a no-op mask unless the tile holds the ragged end
+      }
+    }
+  }
+  const auto l0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
+  float tot = __uint_as_float(l0[0]) + __uint_as_float(l0[1]);
+  uint32_t big = 0;  // the largest magnitude of O's bits: infinities and NaN are 0x7f800000 and up
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    big = max(big, max(__float_as_uint(o[0][r]) & 0x7fffffffu, __float_as_uint(o[1][r]) & 0x7fffffffu));
+  // the sum within [2^-64, 2^64], compared as bits (NaN, too, is outside)
+  constexpr uint32_t LO = 0x1f800000u, HI = 0x5f800000u;
+  if (__syncthreads_or(active && (__float_as_uint(tot) - LO > HI - LO || big >= 0x7f800000u))) {
+    // ---- safe pass (the barrier above also frees the LDS)
+    float q[32];  // channels 32 g + (0..31)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float4 v = load_q(32 * g + 4 * i);
+      q[4 * i] = v.x; q[4 * i + 1] = v.y; q[4 * i + 2] = v.z; q[4 * i + 3] = v.w;
+    }
+    mref = -INFINITY;
+    lsum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { o[0][r] = 0.f; o[1][r] = 0.f; }
+    // DMA: load instruction i (0, 1) of wave w fills tile rows 16 i + 4 w + lane/16; lane slot
+    // lane%16 holds chunk (lane%16) ^ (row & 15) of that row.
+    const int32x4_t rk = make_rsrc_a(Kseq, uint32_t(long(L) * p.ld * 4));
+    const int32x4_t rv = make_rsrc_a(Vseq, uint32_t(long(L) * p.ld * 4));
+    int lrw[2];
+    uint32_t goff[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      lrw[i] = 16 * i + 4 * wave + (lane >> 4);
+      goff[i] = uint32_t(lrw[i] * p.ld * 4 + (((lane & 15) ^ (lrw[i] & 15)) * 16));
+    }
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((lds_cptr_a)smem));
+    const uint32_t tile_bytes = uint32_t(32 * p.ld * 4);
+    auto issue = [&](int t, int B) {
+      const uint32_t so = uint32_t(t) * tile_bytes;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t vo = t * 32 + lrw[i] < L ? goff[i] : 0x80000000u;
+        load_lds_a(rk, vo, so, lds0 + B * TB + (16 * i + 4 * wave) * 256);
+        load_lds_a(rv, vo, so, lds0 + (2 + B) * TB + (16 * i + 4 * wave) * 256);
+      }
+    };
+    const int ks = l32 & 15;  // row swizzle of this lane's K row (row l32)
+    issue(t0, 0);
+    for (int t = t0; t < t1; ++t) {
+      const int B = (t - t0) & 1;
+      wait_vm<0>();  // this wave's share of tile t
+      __syncthreads();  // tile t is in LDS; every wave is past tile t - 1
+      if (t + 1 < t1) issue(t + 1, B ^ 1);
+      if (!active) continue;
+      const char* kb = smem + B * TB;
+      const char* vb = smem + (2 + B) * TB;
+      f32x16 s = {};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // channels 4 i .. 4 i + 3 (+ 32 g)
+        const float4 kf = *reinterpret_cast<const float4*>(kb + l32 * 256 + (((8 * g + i) ^ ks) * 16));
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.x, q[4 * i], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.y, q[4 * i + 1], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.z, q[4 * i + 2], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf.w, q[4 * i + 3], s, 0, 0, 0);
+      }
+      mask(s, t);
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
@@ -853,61 +995,19 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r] - mref);
-    } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r]);
-    }
+      for (int r = 0; r < 16; ++r) lsum += s[r];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lsum += s[r];
-    __builtin_amdgcn_s_setprio(1);
+      for (int dt = 0; dt < 2; ++dt) {
+        const int col = dt * 32 + l32;  // head channel of this lane's V reads
 #pragma unroll
-    for (int dt = 0; dt < 2; ++dt) {
-      const int col = dt * 32 + l32;  // head channel of this lane's V reads
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = 8 * (r >> 2) + 4 * g + (r & 3);
-        const float vf = *reinterpret_cast<const float*>(vb + key * 256 + (((col >> 2) ^ (key & 15)) * 16) + (col & 3) * 4);
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf, s[r], o[dt], 0, 0, 0);
+        for (int r = 0; r < 16; ++r) {
+          const int key = 8 * (r >> 2) + 4 * g + (r & 3);
+          const float vf = *reinterpret_cast<const float*>(vb + key * 256 + (((col >> 2) ^ (key & 15)) * 16) + (col & 3) * 4);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf, s[r], o[dt], 0, 0, 0);
+        }
       }
     }
-    __builtin_amdgcn_s_setprio(0);
-  };
-
-  const int ntiles = (L + 31) / 32;
-  const int t0 = SPLIT ? split * p.tps : 0, t1 = SPLIT ? min(ntiles, t0 + p.tps) : ntiles;
-  const std::integral_constant<int, 0> R0;
-  const std::integral_constant<int, 1> R1;
-  auto pass = [&](auto safe_t) {
-    mref = decltype(safe_t)::value ? -INFINITY : 0.f;
-    lsum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { o[0][r] = 0.f; o[1][r] = 0.f; }
-    issue(t0, R0);
-    wait_vm<0>();
-    __syncthreads();
-    auto step = [&](int t, auto bufc) {
-      constexpr int B = decltype(bufc)::value;
-      issue(t + 1, std::integral_constant<int, B ^ 1>{});  // slot B ^ 1 held tile t-1, done by all
-      if (active) tile(t, bufc, std::false_type{}, safe_t);
-      wait_vm<0>();
-      __syncthreads();
-    };
-    int t = t0;
-    for (; t + 2 < t1; t += 2) {
-      step(t, R0);
-      step(t + 1, R1);
-    }
-    if (t + 1 < t1) step(t++, R0);
-    if (active) {
-      if ((t - t0) & 1) tile(t, R1, std::true_type{}, safe_t);
-      else tile(t, R0, std::true_type{}, safe_t);
-    }
-  };
-  pass(std::false_type{});
-  const auto l0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
-  float tot = __uint_as_float(l0[0]) + __uint_as_float(l0[1]);
-  if (__syncthreads_or(active && !(tot >= 0x1p-64f && tot <= 0x1p64f))) {
-    pass(std::true_type{});
     const auto l1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
     tot = __uint_as_float(l1[0]) + __uint_as_float(l1[1]);
   }
@@ -1013,6 +1113,25 @@ static int attn_splits(long blocks, int ntiles, bool qt2) {
   return best;
 }
 
+// Key slices of an fp32 launch of `blocks` blocks of 128 queries, `ntiles` 32-key tiles each; S <= 8,
+// at least 2 tiles a slice. A CU with n slices takes n x 0.7 of one slice's time (1 for n = 1: two
+// blocks share a CU), a slice its tiles plus about 3 tiles' worth of start, partials and merge.
+// Taken when 5% below the unsplit launch. The partials stay within ATTN_SCRATCH_BYTES, so that the
+// allocation-free entry point takes the same plan. Measured, us for S = 1 .. 8: 1297 tokens x 6
+// heads 71 44 35 37 36 34 32 33; 6 x 973 x 6 82 79 75 78 81 82 85 88; 5838 x 6 412 378 322 319 305
+// 304 303 300; 2593 x 12 139 122 130 127 132 132 135 141; 8 x 1297 x 16 321 330 353 373 391 ...
+static int attn_f32_splits(long blocks, int ntiles, long rows) {
+  int best = 1;
+  double bc = 1e30;
+  for (int S = 1; S <= ATTN_MAX_SPLITS; ++S) {
+    if (S > 1 && (ntiles / S < 2 || size_t(S) * rows * (64 + 2) * sizeof(float) > ATTN_SCRATCH_BYTES)) break;
+    const long n = (blocks * S + 255) / 256;
+    const double cost = (n == 1 ? 1.0 : 0.7 * double(n)) * (double(ntiles) / S + 3.0) * (S > 1 ? 1.05 : 1.0);
+    if (cost < bc * 0.999) { bc = cost; best = S; }
+  }
+  return best;
+}
+
 // The launches of a 16-bit (bf16 or f16) attention: the fast kernel, or the generic one for
 // strides it does not take; then the slice merge when b is split.
 template <typename H>
@@ -1052,9 +1171,7 @@ void attention(const Exec& ex, const AttnArgs& a) {
   auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   const bool f32_fast = a.dt == F32 && long(a.L) * a.ld * 4 < 2147483648L && al16(a.q) && al16(a.k) && al16(a.v) &&
                         al16(a.o);
-  // fp32 (and the generic kernels): one block of 128 queries cannot keep a CU busy (fp32
-  // matrix cores at 1/16 of the bf16 rate), so a small grid is cut into key slices until it
-  // has about two blocks per CU (DA3-Small C1: 66 blocks -> 7 slices).
+  // The generic kernels cut a small grid into key slices until it has about two blocks per CU.
   const long gblocks = long(cdiv(a.L, ATTN_WAVES * 32)) * a.heads * a.seqs;
   // 4 waves x 32 or 64 queries. Two query sub-tiles per wave (QT = 2) halve the K/V reads per
   // query; four QT=1 or two QT=2 blocks fit a CU. Unsplit launches (L < 4096) take QT = 2 when
@@ -1075,10 +1192,10 @@ void attention(const Exec& ex, const AttnArgs& a) {
     qt2 = u2 < u1 || (u2 == u1 && blocks2 >= 256);
   }
   const long blocks = qt2 ? blocks2 : blocks1;
-  // the fp32 kernel's 32-key tiles: slices of at least 4 tiles, about two blocks per CU
+  // (the fp32 kernel's tiles have 32 keys)
   const int ntiles = f32_fast ? cdiv(a.L, 32) : cdiv(a.L, 64);
   int S = bf_fast    ? (a.L >= 4096 ? attn_splits(blocks, ntiles, qt2) : 1)
-                : f32_fast ? int(std::min<long>(std::min<long>(8, std::max(1, ntiles / 4)), std::max<long>(1, cdiv(512, gblocks))))
+                : f32_fast ? attn_f32_splits(gblocks, ntiles, long(a.seqs) * a.L * a.heads)
                            : int(std::min<long>(std::min<long>(8, ntiles / 2), std::max<long>(1, cdiv(512, gblocks))));
   // Tail split: a grid past whole rounds of 256 blocks runs those rounds whole and only the tail
   // in key slices, so that each CU gets about the same work without every block paying for

@@ -1,4 +1,4 @@
-"""fp32 products from three bf16 parts (gemm, convolutions) against float64: sizes at the
+"""fp32 products from three bf16 parts (gemm, convolutions, attention) against float64: sizes at the
 edges of the tiles, wide ranges, and operands that are infinite, NaN or round to infinity in bf16.
 
 Tolerance (2-norm of the error over the result's): the parts are exact and the products left out are
@@ -112,3 +112,47 @@ def test_conv_matches_float64(ctx, V, H, W, C, N, relu):
     err = float((out.cpu().double() - ref).norm() / ref.norm())
     report("f32.conv", V=V, H=H, W=W, C=C, N=N, err=f"{err:.2e}")
     assert err <= _tol(9 * C)
+
+
+def _attention(ctx, qkv, S, L, heads):
+    out = torch.full((S * L, heads * 64), -7.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_attention(splathip.F32, qkv.data_ptr(), out.data_ptr(), S, L, heads)
+    ctx.synchronize()
+    return out.cpu().double().reshape(S, L, heads, 64).permute(0, 2, 1, 3)
+
+
+def _attention_ref(qkv, S, L, heads):
+    q, k, v = qkv.cpu().double().reshape(S, L, 3, heads, 64).permute(2, 0, 3, 1, 4)
+    return torch.softmax(q @ k.transpose(-1, -2) / 8, -1) @ v
+
+
+@pytest.mark.parametrize("S,L,heads", [(1, 1, 1), (2, 31, 2), (1, 33, 3), (3, 64, 1), (2, 129, 2), (1, 257, 6),
+                                       (1, 1297, 6), (2, 700, 3)])
+def test_attention_matches_float64(ctx, S, L, heads):
+    """The scores' roundings reach the weights as they are, the weighted sum takes six for every 16
+    keys: within 2^-24 (sqrt(6 L / 16) + 64), the 64 for scores up to about 8 and the exponential."""
+    g = torch.Generator().manual_seed(L)
+    qkv = _rand(g, S * L, 3 * heads * 64)
+    out, ref = _attention(ctx, qkv, S, L, heads), _attention_ref(qkv, S, L, heads)
+    err = float((out - ref).norm() / ref.norm())
+    report("f32.attention", S=S, L=L, heads=heads, err=f"{err:.2e}")
+    assert err <= 2.0 ** -24 * ((6 * max(L, 16) / 16) ** 0.5 + 64)
+
+
+def test_attention_special_values(ctx):
+    """An infinite value reaches its channel of every query and no other."""
+    S, L, heads = 1, 300, 2
+    g = torch.Generator().manual_seed(2)
+    qkv = _rand(g, S * L, 3 * heads * 64)
+    v = qkv.view(L, 3, heads, 64)[:, 2]
+    v[17, 0, 5] = float("inf")
+    v[290, 0, 40] = float("-inf")
+    out = _attention(ctx, qkv, S, L, heads)
+    ref = _attention_ref(qkv, S, L, heads)
+    report("f32.attention.special", inf=int(torch.isinf(out).sum()), ref=int(torch.isinf(ref).sum()),
+           nan=int(torch.isnan(out).sum()))
+    assert torch.equal(torch.isinf(out), torch.isinf(ref)) and not torch.isnan(out).any()
+    assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
+    fine = torch.isfinite(ref)
+    assert float(((out[fine] - ref[fine]).abs() / (ref[fine].abs() + 1.0)).max()) < 1e-5
