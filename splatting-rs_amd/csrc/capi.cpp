@@ -566,10 +566,15 @@ int splat_kernel_reconstruct(splat_ctx* ctx, int V, int H, int W, const float* d
   return guard(c, [&] {
     SPLAT_CHECK(V > 0 && H > 0 && W > 0 && conf && cameras && points && conf_out, BAD_ARGUMENT, "geometry args");
     const size_t px = size_t(V) * H * W;
-    float* d_conf0 = static_cast<float*>(staging(c, 21, px * 4));
+    // the cleaning compares the given confidences of other pixels: in place, it reads a copy
+    if (conf < conf_out + px && conf_out < conf + px) {
+      float* copy = static_cast<float*>(staging(c, 21, px * 4));
+      convert(c->ex, F32, conf, F32, copy, long(px));
+      conf = copy;
+    }
     double* d_fit = depth ? nullptr : static_cast<double*>(staging(c, 24, size_t(V) * 4 * 8));
     reconstruct_geometry(c->ex, V, H, W, depth, pose_encoding, points_in_camera, quaternion, translation, conf, mask,
-                         foreground, cameras, d_fit, d_conf0, points, conf_out);
+                         foreground, cameras, d_fit, points, conf_out);
   });
 }
 
@@ -695,14 +700,13 @@ int splat_da3_reconstruct(splat_ctx* ctx, const float* images, int V, int H, int
     dev.pose_encoding = static_cast<float*>(staging(c, 4, V * 9 * 4));
     int32_t* d_ref = static_cast<int32_t*>(staging(c, 6, 4));
     double* d_cam = static_cast<double*>(staging(c, 20, size_t(V) * 16 * 8));
-    float* d_conf0 = static_cast<float*>(staging(c, 21, px * 4));
     float* d_points = static_cast<float*>(staging(c, 22, px * 12));
     float* d_conf = static_cast<float*>(staging(c, 23, px * 4));
     SPLAT_HIP(hipMemcpyAsync(d_img, images, px * 3 * 4, hipMemcpyHostToDevice, c->stream));
     const uint8_t* d_fg = stage_foreground(c, foreground, px);
     da3_device(c, d_img, V, H, W, dev, d_ref);
     reconstruct_geometry(c->ex, V, H, W, dev.depth, dev.pose_encoding, nullptr, nullptr, nullptr, dev.depth_conf,
-                         nullptr, d_fg, d_cam, nullptr, d_conf0, d_points, d_conf);
+                         nullptr, d_fg, d_cam, nullptr, d_points, d_conf);
     int32_t ref = 0;
     SPLAT_HIP(hipMemcpyAsync(&ref, d_ref, 4, hipMemcpyDeviceToHost, c->stream));
     std::vector<float> pose(size_t(V) * 9), depth(px);
@@ -739,7 +743,6 @@ int splat_ma_reconstruct(splat_ctx* ctx, const float* images, int V, int H, int 
     dev.conf = static_cast<float*>(staging(c, 16, px * 4));
     dev.mask = static_cast<uint8_t*>(staging(c, 17, px));
     double* d_cam = static_cast<double*>(staging(c, 20, size_t(V) * 16 * 8));
-    float* d_conf0 = static_cast<float*>(staging(c, 21, px * 4));
     float* d_points = static_cast<float*>(staging(c, 22, px * 12));
     float* d_conf = static_cast<float*>(staging(c, 23, px * 4));
     double* d_fit = static_cast<double*>(staging(c, 24, size_t(V) * 4 * 8));
@@ -747,7 +750,7 @@ int splat_ma_reconstruct(splat_ctx* ctx, const float* images, int V, int H, int 
     const uint8_t* d_fg = stage_foreground(c, foreground, px);
     ma_device(c, d_img, V, H, W, dev, nullptr, false, intrinsics);
     reconstruct_geometry(c->ex, V, H, W, nullptr, nullptr, dev.points, dev.quaternion, dev.translation, dev.conf,
-                         dev.mask, d_fg, d_cam, d_fit, d_conf0, d_points, d_conf);
+                         dev.mask, d_fg, d_cam, d_fit, d_points, d_conf);
     recon_outputs(c, V, H, W, d_cam, d_points, d_conf, dev.points + 2, 3, out);
     out->reference_view = 0;
   });

@@ -194,11 +194,11 @@ void add_view_features(const Exec& ex, float* xs, int V, int n, int P, int dim, 
 // pose_enc [V,9]; MapAnything (depth NULL): camera-frame points pts_cam [V,H,W,3], xyzw quat
 // [V,4], metric trans [V,3], unambiguous mask, fitted [V,4] scratch. conf [V,H,W] in;
 // fg [V,H,W] foreground (NULL = all). Out: cam [V,16] (R row-major, t, fx, fy, cx, cy in
-// view 0's frame), conf0 scratch, points [V,H,W,3] in view 0's frame, cleaned conf_out.
+// view 0's frame), points [V,H,W,3] in view 0's frame, cleaned conf_out (not over conf).
 void reconstruct_geometry(const Exec& ex, int V, int H, int W, const float* depth, const float* pose_enc,
                           const float* pts_cam, const float* quat, const float* trans, const float* conf,
-                          const uint8_t* mask, const uint8_t* fg, double* cam, double* fitted, float* conf0,
-                          float* points, float* conf_out);
+                          const uint8_t* mask, const uint8_t* fg, double* cam, double* fitted, float* points,
+                          float* conf_out);
 
 // RGBA u8 [V,H,W,4] -> normalised images [V,3,H,W] f32 and foreground [V,H,W] (NULL: skipped).
 void to_model_input(const Exec& ex, const uint8_t* rgba, int V, int H, int W, float* img, uint8_t* fg);
