@@ -555,6 +555,7 @@ Context::~Context() {
   (void)hipSetDevice(device);
   if (stream) (void)hipStreamSynchronize(stream);
   if (aux) (void)hipStreamSynchronize(aux);
+  ring_.reset();
   clear_graphs();
   da3.reset();
   ma.reset();
@@ -579,6 +580,32 @@ void* Context::staging_buffer(int slot, size_t bytes) {
     s.second = bytes;
   }
   return s.first;
+}
+
+HostRing::HostRing() {
+  try {
+    SPLAT_HIP(hipHostMalloc(reinterpret_cast<void**>(&base), SLOTS * CHUNK, hipHostMallocDefault));
+    for (hipEvent_t& e : sent) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (hipEvent_t& e : copied) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (hipEvent_t& e : used) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  } catch (...) {
+    this->~HostRing();
+    throw;
+  }
+}
+
+HostRing::~HostRing() {
+  for (hipEvent_t* e : {&sent[0], &copied[0], &used[0]}) {
+    const int n = e == &sent[0] ? SLOTS : 2;
+    for (int k = 0; k < n; ++k)
+      if (e[k]) (void)hipEventDestroy(e[k]);
+  }
+  if (base) (void)hipHostFree(base);
+}
+
+HostRing& Context::host_ring() {
+  if (!ring_) ring_ = std::make_unique<HostRing>();
+  return *ring_;
 }
 
 void Context::clear_graphs() {

@@ -293,6 +293,18 @@ class MaModel {
 
 // --- context ---------------------------------------------------------------------------------
 
+// Pinned host memory that pageable photos go to the GPU through, in chunks, several threads filling
+// it (one thread copies at about half the link's rate): SLOTS chunks in flight. `sent`: a slot's
+// copy; `copied` / `used`: a photo's device buffer written / read (two of them in turn).
+struct HostRing {
+  static constexpr size_t CHUNK = size_t(2) << 20;
+  static constexpr int SLOTS = 8, THREADS = 3;
+  uint8_t* base = nullptr;
+  hipEvent_t sent[SLOTS] = {}, copied[2] = {}, used[2] = {};
+  HostRing();
+  ~HostRing();
+};
+
 class Context {
  public:
   explicit Context(int device);
@@ -330,6 +342,10 @@ class Context {
   // Grow-only device buffers the host-pointer entry points stage inputs/outputs in.
   std::map<int, std::pair<void*, size_t>> staging;
   void* staging_buffer(int slot, size_t bytes);
+
+  // The pinned ring of the photo uploads, allocated on first use.
+  HostRing& host_ring();
+  std::unique_ptr<HostRing> ring_;
 
   // Graph cache: key -> instantiated graph.
   struct GraphKey {
