@@ -1600,12 +1600,15 @@ static BfShape bf_shape(BfCfg c) {
 // fp32 (64x64 tiles): at most 160 tiles, one round of slices of at least 6 k-tiles or two rounds of at
 // least 12 (us unsplit / split, the reduce included: 1297x384x1536 126 tiles 31.6 / 22.4 in 4; 3x3 of 64
 // channels, K = 576: 81 tiles 16.8 / 14.2 in 3, 21 tiles 16.2 / 12.1 in 3; 324 tiles lose, 26.2 / 29.7).
+// The two larger fp32 tiles never split: they are taken where 64x64 tiles already fill the chip (162 tiles
+// of 128x64, K = 576: 32.9 in 2 with the reduce, 23.5 as 324 tiles of 64x64 unsplit).
 static int split_factor(const GemmArgs& a, BfCfg c) {
   if (a.hw3 || a.ln_in) return 1;  // the fused head needs whole tiles, a folded LayerNorm whole rows of K
   const BfShape sh = bf_shape(c);
   const long tiles = long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn);
   const long slots = long(GEMM_CUS) * sh.per_cu;
   const int nk = cdiv(a.K, a.dt == F32 ? 32 : 64);
+  if (c == CFG_F128x128 || c == CFG_F128x64) return 1;
   int S;
   if (c == CFG_F64x64) {
     if (tiles > 160) return 1;
@@ -1634,7 +1637,7 @@ static size_t split_bytes(const GemmArgs& a, int S) {
   if (a.N <= 32 && !a.qk_dim) return CFG_128x32;
   if (split_factor(a, CFG_F64x64) > 1) return CFG_F64x64;
   const BfCfg cands[] = {CFG_F128x128, CFG_F128x64, CFG_F64x64};
-  const double eff[] = {1.0, 0.82, 0.69}, alone[] = {1.0, 1.15, 1.15};
+  const double eff[] = {1.0, 0.82, 0.69}, alone[] = {1.0, 1.2, 1.15};
   double best = 1e30;
   BfCfg pick = CFG_F128x128;
   for (int i = 0; i < 3; ++i) {
