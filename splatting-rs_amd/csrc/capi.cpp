@@ -572,6 +572,12 @@ int splat_kernel_reconstruct(splat_ctx* ctx, int V, int H, int W, const float* d
       convert(c->ex, F32, conf, F32, copy, long(px));
       conf = copy;
     }
+    // and other pixels' depths: points over the points they come from
+    if (points_in_camera && points_in_camera < points + 3 * px && points < points_in_camera + 3 * px) {
+      float* copy = static_cast<float*>(staging(c, 22, px * 12));
+      convert(c->ex, F32, points_in_camera, F32, copy, long(px) * 3);
+      points_in_camera = copy;
+    }
     double* d_fit = depth ? nullptr : static_cast<double*>(staging(c, 24, size_t(V) * 4 * 8));
     reconstruct_geometry(c->ex, V, H, W, depth, pose_encoding, points_in_camera, quaternion, translation, conf, mask,
                          foreground, cameras, d_fit, points, conf_out);

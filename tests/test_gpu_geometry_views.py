@@ -43,3 +43,32 @@ def test_views(ctx, V, H, W, in_place):
     differ = float(np.mean(out.cpu().numpy() != ref["conf"]))
     report("geometry.views", V=V, in_place=in_place, differ=differ, zeroed=float(np.mean(ref["conf"] == 0)))
     assert differ <= 1e-3
+
+
+def test_points_over_their_source(ctx):
+    """MapAnything's points written over the camera-frame points: what separate buffers give."""
+    V, H, W = 4, 70, 98
+    g = torch.Generator().manual_seed(1)
+    y, x = torch.meshgrid(torch.linspace(-0.4, 0.4, H), torch.linspace(-0.5, 0.5, W), indexing="ij")
+    z = 2 + 0.1 * torch.randn(V, H, W, generator=g)
+    pts = torch.stack([x * z, y * z, z], -1).cuda()
+    quat = torch.tensor([[0.0, 0.0, 0.0, 1.0]]).repeat(V, 1).cuda()
+    trans = torch.randn(V, 3, generator=g).mul(0.05).cuda()
+    trans[:, 2] -= 0.5 * torch.arange(V).cuda()   # the views' depths differ from view 0's
+    conf = (1 + torch.exp(torch.randn(V, H, W, generator=g))).cuda()
+    mask = (torch.rand(V, H, W, generator=g) < 0.9).to(torch.uint8).cuda()
+
+    def call(source, points):
+        cams, out = torch.empty(V, 16, dtype=torch.float64, device="cuda"), torch.empty_like(conf)
+        torch.cuda.synchronize()
+        ctx.kernel_reconstruct(V, H, W, points_in_camera=source.data_ptr(), quaternion=quat.data_ptr(),
+                               translation=trans.data_ptr(), conf=conf.data_ptr(), mask=mask.data_ptr(),
+                               cameras=cams.data_ptr(), points=points.data_ptr(), conf_out=out.data_ptr())
+        ctx.synchronize()
+        return cams, points, out
+
+    ref = call(pts, torch.empty_like(pts))
+    both = pts.clone()
+    got = call(both, both)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    assert 0 < int((ref[2] == 0).sum()) < conf.numel()
