@@ -1657,7 +1657,10 @@ static bool launch_f32_auto(const Exec& ex, const GemmArgs& a) {
   if (S > 1 && !(ex.ws && ex.ws->ptr && ex.ws->cap >= split_bytes(a, S))) S = 1;
   switch (c) {
     case CFG_128x32: return launch_mfma<T, 128, 32, 4, 1, 2>(ex, a, S);
-    case CFG_F128x128: return launch_mfma<T, 128, 128, 2, 2, 2>(ex, a, S);
+    // two blocks a CU enforced: left alone, the everything-else epilogue (EPI_FULL) took 64 registers
+    // more, one block (us, one block -> two: 3x3 of 128 channels with ReLU on load and residual on 93312
+    // pixels 209 -> 174; 4x4 transposed convolution of 256 channels on 6 x 28x37 137 -> 106)
+    case CFG_F128x128: return launch_mfma<T, 128, 128, 2, 2, 2, 32, 2>(ex, a, S);
     case CFG_F128x64: return launch_mfma<T, 128, 64, 2, 2, 2>(ex, a, S);
     default: return launch_mfma<T, 64, 64, 2, 2, 2>(ex, a, S);
   }
