@@ -792,6 +792,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
 
   f32x16 o[2];
   float mref = 0.f, lsum = 0.f;
+  uint32_t lost = 0;  // what the splits of Q, K and V cut
 #pragma unroll
   for (int r = 0; r < 16; ++r) { o[0][r] = 0.f; o[1][r] = 0.f; }
   // keys past L in the last tile weigh nothing
@@ -817,7 +818,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
     for (int st = 0; st < 4; ++st) {
       const float4 a = load_q(16 * st + 8 * g), b = load_q(16 * st + 8 * g + 4);
       const float w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      q[st] = split8(w);
+      q[st] = split8<true>(w, lost);
     }
     // this thread's part of a tile: key row tid / 8, channels 8 (tid % 8) + (0..7)
     const int trow = tid >> 3, tch = tid & 7;
@@ -839,7 +840,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
     };
     auto store = [&](int buf) {
       char* kb = smem + buf * KVB;
-      const Split8 k = split8(rk[0], rk[1]), v = split8(rv[0], rv[1]);
+      const Split8 k = split8<true>(rk[0], rk[1], lost), v = split8<true>(rv[0], rv[1], lost);
       *reinterpret_cast<uint4*>(kb + kdst) = k.h;
       *reinterpret_cast<uint4*>(kb + PB + kdst) = k.m;
       *reinterpret_cast<uint4*>(kb + 2 * PB + kdst) = k.l;
@@ -892,7 +893,7 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
         float w[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) w[e] = s[8 * hh + e];
-        const Split8 ps = split8(w);
+        const Split8 ps = split8<false>(w, lost);  // a weight's last bits below 2^-133 are below 2^-69 of the sum
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int dt = 0; dt < 2; ++dt) {
@@ -926,7 +927,8 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
     big = max(big, max(__float_as_uint(o[0][r]) & 0x7fffffffu, __float_as_uint(o[1][r]) & 0x7fffffffu));
   // the sum within [2^-64, 2^64], compared as bits (NaN, too, is outside)
   constexpr uint32_t LO = 0x1f800000u, HI = 0x5f800000u;
-  if (__syncthreads_or(active && (__float_as_uint(tot) - LO > HI - LO || big >= 0x7f800000u))) {
+  if (__syncthreads_or((lost & SPLIT_LOST) ||
+                       (active && (__float_as_uint(tot) - LO > HI - LO || big >= 0x7f800000u)))) {
     // ---- safe pass (the barrier above also frees the LDS)
     float q[32];  // channels 32 g + (0..31)
 #pragma unroll

@@ -202,14 +202,18 @@ __host__ __device__ inline int xcd_contiguous(int b, int nblk) {
   const int x = b & 7, q8 = nblk >> 3, r8 = nblk & 7;
   return (x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8) + (b >> 3);
 }
-// Eight floats as three bf16 vectors, x = h + m + l exactly: h and m are the value and the
-// remainder rounded to nearest, so |m| <= 2^-9 |x|, |l| <= 2^-18 |x|, and 24 significant bits
-// leave at most 8 for l. 44 instructions that all run beside the matrix cores (v_dot2_f32_bf16
-// would take a remainder from the packed pair in one, but it occupies the matrix pipe: five of
-// them after an MFMA cost 33 cycles, five subtractions 2). Not finite: NaN (infinities, and
-// values that round to one): callers take such sums again from the operands as they are.
+// Eight floats as three bf16 vectors, x = h + m + l: h and m are the value and the remainder
+// rounded to nearest, so |m| <= 2^-9 |x|, |l| <= 2^-18 |x|, and 24 significant bits leave at most 8
+// for l: exact from 2^-110 up. Below, the last bits of x lie under bf16's smallest subnormal, 2^-133,
+// and l is cut: then `lost` has a bit set in its lower half. Infinities, and values that round to one
+// in bf16, become NaN. In both cases callers take the sums again from the operands as they are.
+// 44 instructions, 48 with CHECK, that all run beside the matrix cores (v_dot2_f32_bf16 would take
+// a remainder from the packed pair in one, but it occupies the matrix pipe: five of them after an
+// MFMA cost 33 cycles, five subtractions 2).
 struct Split8 { uint4 h, m, l; };
-__device__ inline Split8 split8(const float (&x)[8]) {
+constexpr uint32_t SPLIT_LOST = 0xffffu;
+template <bool CHECK>
+__device__ inline Split8 split8(const float (&x)[8], uint32_t& lost) {
   uint32_t o[3][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -221,14 +225,19 @@ __device__ inline Split8 split8(const float (&x)[8]) {
       b -= __uint_as_float(o[q][i] & 0xffff0000u);
     }
     o[2][i] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);  // the upper halves
+    if constexpr (CHECK) {
+      lost |= __float_as_uint(a) | __float_as_uint(b);
+      asm("" : "+v"(lost));  // taken here: the compiler would keep every remainder for one tree of ors
+    }
   }
   return {make_uint4(o[0][0], o[0][1], o[0][2], o[0][3]), make_uint4(o[1][0], o[1][1], o[1][2], o[1][3]),
           make_uint4(o[2][0], o[2][1], o[2][2], o[2][3])};
 }
-__device__ inline Split8 split8(const uint4& lo, const uint4& hi) {
+template <bool CHECK>
+__device__ inline Split8 split8(const uint4& lo, const uint4& hi, uint32_t& lost) {
   const float x[8] = {__uint_as_float(lo.x), __uint_as_float(lo.y), __uint_as_float(lo.z), __uint_as_float(lo.w),
                       __uint_as_float(hi.x), __uint_as_float(hi.y), __uint_as_float(hi.z), __uint_as_float(hi.w)};
-  return split8(x);
+  return split8<CHECK>(x, lost);
 }
 #endif
 

@@ -831,13 +831,14 @@ constexpr uint32_t OOB = 0x80000000u;
 // at most 32 taps (chosen by the launcher; callers pass A_CONV): each k-tile lies in one tap.
 constexpr int A_CONV_TAP = 2;
 
-// An fp32 wave whose sums are not all finite takes them again from the operands as they are, on
-// v_mfma_f32_32x32x2_f32: split8 turns an infinity (and a value that rounds to one in bf16) into
-// NaN, which must not reach outputs that are infinite or finite. Rows of A or W past the operand
-// are zeros, as in the main loop. Rare, so it reads global memory without staging.
+// An fp32 wave whose sums are not all finite, or one of whose operands split8 cut, takes its sums
+// again from the operands as they are, on v_mfma_f32_32x32x2_f32: split8 turns an infinity (and a
+// value that rounds to one in bf16) into NaN, which must not reach outputs that are infinite or
+// finite. Rows of A or W past the operand are zeros, as in the main loop. Rare, so it reads global
+// memory without staging.
 template <int TM, int TN, bool CONV, bool RELU>
-__device__ inline void plain_products(const GemmArgs& p, f32x16 (&acc)[TM][TN], long wrow0, long wcol0, int k0, int k1,
-                                      int lane) {
+__device__ inline void plain_products(const GemmArgs& p, f32x16 (&acc)[TM][TN], bool cut, long wrow0, long wcol0,
+                                      int k0, int k1, int lane) {
   float t = 0.f;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -845,7 +846,7 @@ __device__ inline void plain_products(const GemmArgs& p, f32x16 (&acc)[TM][TN], 
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) t = fmaf(acc[i][j][r], 0.f, t);  // NaN once a sum is not finite
-  if (!__any(t != 0.f)) return;
+  if (!__any(t != 0.f || cut)) return;
   const int g = lane >> 5, l32 = lane & 31;
   const float* A = reinterpret_cast<const float*>(p.A);
   const float* W = reinterpret_cast<const float*>(p.W);
@@ -976,6 +977,9 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
   // and its offset are uniform; each row keeps a bit mask of its in-bounds taps and its byte
   // offset at tap (0, 0) (modulo 2^32: the sum with a valid tap's offset is the real offset).
   constexpr bool conv_fast = AMODE == A_CONV_TAP;
+  // The fp32 per-lane path takes the mask and the offset too (three registers a row fewer than the
+  // coordinates: the 128x128 tile keeps two blocks a CU without spills).
+  constexpr bool conv_mask = conv_fast || (AMODE == A_CONV && F32T);
   uint32_t tmsk[AL], rbase[AL];
   if (AMODE == A_ROWS) {
     ra = make_rsrc(p.A, uint32_t(long(p.M) * p.lda * ES));
@@ -1003,7 +1007,7 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
       }
       tmsk[i] = 0;
       rbase[i] = 0;
-      if (conv_fast && m < p.M) {
+      if (conv_mask && m < p.M) {
         rbase[i] = aoff[i] + uint32_t(((long(aiy[i]) * p.Wi + aix[i]) * p.Cin + c * KE) * ES);
         for (int ky = 0; ky < p.ks; ++ky)
           for (int kx = 0; kx < p.ks; ++kx) {
@@ -1050,6 +1054,13 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
       } else {
         const int tap = k / p.Cin, ci = k - tap * p.Cin;
         const int ky = tap / p.ks, kx = tap - ky * p.ks;
+        if constexpr (conv_mask) {
+          // as above, without a branch: bit 31 for a tap out of bounds or a chunk past kend
+          const uint32_t bad = (((tmsk[i] >> (tap & 31)) & 1u) ^ 1u) | uint32_t(!kin);
+          load_to_lds(ra, (rbase[i] + uint32_t(((ky * p.Wi + kx) * p.Cin + ci - c * KE) * ES)) | (bad << 31), 0u,
+                      sb + (i * NW + wave) * 1024);
+          return;
+        }
         const int iy = aiy[i] + ky, ix = aix[i] + kx;
         const bool ok = kin && iy >= 0 && iy < p.Hi && ix >= 0 && ix < p.Wi;
         load_to_lds(ra, ok ? aoff[i] + uint32_t((iy * p.Wi + ix) * p.Cin + ci) * ES : OOB, 0u,
@@ -1069,7 +1080,12 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  const int sw = (l32 >> SH) & (CPR - 1);
+  // fp32 tiles of 2 x 2 waves: the two waves that share an operand fragment walk the two k-steps
+  // of a tile in opposite order, so that each checks its first (split_frag) and both together everything
+  constexpr bool SHARED_CHECK = F32T && WM == 2 && WN == 2;
+  float* any_cut = LdsFloats<SHARED_CHECK ? 1 : 0>::get();
+  if (SHARED_CHECK && tid == 0) *any_cut = 0.f;  // before the first barrier
+  const int sw = ((l32 >> SH) & (CPR - 1)) ^ (SHARED_CHECK ? ((wm ^ wn) & 1) << 2 : 0);
   const int arow0 = (wm * (BM / WM) + l32) * RB, brow0 = (BM + wn * (BN / WN) + l32) * RB;
   // byte offset of this lane's chunk h in k-step s of a tile row
   auto step_off = [&](int st, int h) { return (((FH * st + h) * 2 + g) ^ sw) * 16; };
@@ -1132,6 +1148,7 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
   // Fragments of the next k-step (of this tile, or step 0 of the next tile) are read while the
   // matrix cores work on the current one.
   uint4 fa[2][TM * FH], fb[2][TN * FH];
+  [[maybe_unused]] uint32_t lost = 0;  // fp32: what the splits cut
   // Fragment f of a k-step in the order the MFMAs (i outer, j inner) first use them: the A
   // fragments of tile row 0, then every W fragment, then the other A ones, so that the first
   // MFMAs of a step wait for few reads. Fragment f: chunk f % FH of 32-row tile f / FH.
@@ -1168,24 +1185,26 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
 #pragma unroll
       for (int j = 0; j < (LOW ? TN : 1); ++j) low[i][j] = f32x16{};
     constexpr int MM = TM * TN, NF = (TM + TN) * FH, NS = TM + TN;
-    constexpr int SV = (NS * 44 / MM + 5) / 6;  // VALU instructions of the splits after each MFMA
+    constexpr int SV = ((NS * (SHARED_CHECK ? 46 : 48) + (RELU ? TM * 8 : 0)) / MM + 5) / 6;  // VALU of the splits after each MFMA
     // fragments of `slot` -> parts of the same k-step parity
-    auto split_frag = [&](int slot, int f) {
+    auto split_frag = [&](auto slot_c, int f) {
+      constexpr int slot = decltype(slot_c)::value;
+      constexpr bool CHECK = !SHARED_CHECK || slot == 0;
       if (f < TN) {
-        pb[slot][f] = split8(fb[slot][2 * f], fb[slot][2 * f + 1]);
+        pb[slot][f] = split8<CHECK>(fb[slot][2 * f], fb[slot][2 * f + 1], lost);
       } else {
         uint4 x = fa[slot][2 * (f - TN)], y = fa[slot][2 * (f - TN) + 1];
         if (RELU) {
           x = Mfma<float>::relu(x);
           y = Mfma<float>::relu(y);
         }
-        pa[slot][f - TN] = split8(x, y);
+        pa[slot][f - TN] = split8<CHECK>(x, y, lost);
       }
     };
     read_frags(0, 0, 0);
     read_frags(0, 1, 1);
 #pragma unroll
-    for (int f = 0; f < NS; ++f) split_frag(0, f);
+    for (int f = 0; f < NS; ++f) split_frag(std::integral_constant<int, 0>{}, f);
     auto tile = [&](int kt, auto has_next, auto full) {
       constexpr bool HAS_NEXT = decltype(has_next)::value;
       if constexpr (HAS_NEXT) {
@@ -1208,7 +1227,10 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
           }
           if (HAS_NEXT || s == 0) {
 #pragma unroll
-            for (int f = q * NS / MM; f < (q + 1) * NS / MM; ++f) split_frag(s ^ 1, f);
+            for (int f = q * NS / MM; f < (q + 1) * NS / MM; ++f) {
+              if (s == 0) split_frag(std::integral_constant<int, 1>{}, f);
+              else split_frag(std::integral_constant<int, 0>{}, f);
+            }
           }
           f32x16& c = acc[q / TN][q % TN];
           Mfma<float>::mma_split(c, LOW ? low[LOW ? q / TN : 0][LOW ? q % TN : 0] : c, pa[s][q / TN], pb[s][q % TN]);
@@ -1309,7 +1331,11 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
     tile(nk - 1, std::false_type{}, std::false_type{});
   }
   wait_vmcnt<0>();  // the zero-fill loads past the last tile must land before the ring is reused
-  __syncthreads();  // every wave is past its last read of the ring before slabs reuse it
+  // every wave is past its last read of the ring before slabs reuse it
+  bool cut = (lost & SPLIT_LOST) != 0;  // an operand of the wave (of the tile) was cut by a split
+  if (SHARED_CHECK && cut) *any_cut = 1.f;
+  __syncthreads();
+  if (SHARED_CHECK) cut = *any_cut != 0.f;
   if constexpr (SPLITR && EPI == EPI_LN) {
     if (tid < BM) {
       lnab[2 * tid] = ln_rstd;
@@ -1319,7 +1345,8 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
   }
   if constexpr (F32T) {
     __builtin_amdgcn_s_setprio(0);
-    plain_products<TM, TN, AMODE != A_ROWS, RELU>(p, acc, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kt0 * BK, kend, lane);
+    plain_products<TM, TN, AMODE != A_ROWS, RELU>(p, acc, cut, m0 + wm * (BM / WM), n0 + wn * (BN / WN), kt0 * BK,
+                                                  kend, lane);
   }
   if constexpr (EPI == EPI_HEAD) {
     static_assert(NW * 32 * slab_ld(TN) * 4 + BM * WN * 6 * 4 <= RING, "head epilogue LDS");

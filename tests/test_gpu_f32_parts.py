@@ -1,5 +1,6 @@
 """fp32 products from three bf16 parts (gemm, convolutions, attention) against float64: sizes at the
-edges of the tiles, wide ranges, and operands that are infinite, NaN or round to infinity in bf16.
+edges of the tiles, wide ranges down to fp32's smallest normal number, and operands that are infinite, NaN or
+round to infinity in bf16.
 
 Tolerance (2-norm of the error over the result's): the parts are exact and the products left out are
 below 3 * 2^-26; what is left are the roundings of the sum, at most six for every 16 values of K, each
@@ -64,6 +65,37 @@ def test_gemm_wide_range(ctx, exp):
     scale = A.double().norm(dim=1)[:, None] * W.double().norm(dim=1)[None]
     err = float(((out - ref) / scale).norm() / (ref / scale).norm())
     assert err <= _tol(256)
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 96, 256), (140, 64, 1536), (70, 96, 128), (2100, 1152, 64)])
+@pytest.mark.parametrize("side", ["a", "w"])
+def test_gemm_tiny_values(ctx, M, N, K, side):
+    """One operand's rows (of A, or of W) lie at 2^-126 to 2^-90, where the third part of a split falls under
+    bf16's smallest subnormal; the other operand brings the results back to ordinary sizes. Every
+    row is right by itself: the fp32 instructions keep all 24 bits there."""
+    g = torch.Generator().manual_seed(M + K)
+    A, W = _rand(g, M, K), _rand(g, N, K)
+    small, big = (A, W) if side == "a" else (W, A)
+    e = torch.linspace(-124, -90, small.shape[0]).floor()
+    small.mul_(torch.exp2(e)[:, None].cuda())
+    small[small.abs() < 2.0 ** -126] = 0.0
+    big.mul_(2.0 ** 100)
+    out = _gemm(ctx, A, W, torch.zeros(N, device="cuda")).double()
+    ref = A.double() @ W.double().t()
+    dim = 1 if side == "a" else 0
+    err = ((out - ref).norm(dim=dim) / ref.norm(dim=dim)).max()
+    report("f32.tiny", M=M, N=N, K=K, side=side, err=f"{float(err):.2e}")
+    assert float(err) <= 2 * _tol(K)   # the worst row, not the whole matrix
+
+
+def test_gemm_few_tiny_values(ctx):
+    """Ordinary operands with a tiny value here and there: the waves that redo their sums agree."""
+    g = torch.Generator().manual_seed(4)
+    A, W = _rand(g, 300, 384), _rand(g, 200, 384)
+    A[::7, 3], W[::5, 9] = 1.2345e-37, -3.21e-36
+    out = _gemm(ctx, A, W, torch.zeros(200, device="cuda")).double()
+    ref = A.double() @ W.double().t()
+    assert float((out - ref).norm() / ref.norm()) <= _tol(384)
 
 
 def _same(out, ref, tol):
@@ -137,6 +169,25 @@ def test_attention_matches_float64(ctx, S, L, heads):
     out, ref = _attention(ctx, qkv, S, L, heads), _attention_ref(qkv, S, L, heads)
     err = float((out - ref).norm() / ref.norm())
     report("f32.attention", S=S, L=L, heads=heads, err=f"{err:.2e}")
+    assert err <= 2.0 ** -24 * ((6 * max(L, 16) / 16) ** 0.5 + 64)
+
+
+@pytest.mark.parametrize("S,L,heads", [(1, 40, 2), (1, 1297, 2)])   # unsplit; key slices
+@pytest.mark.parametrize("which", ["k", "v"])
+def test_attention_tiny_values(ctx, S, L, heads, which):
+    """K at 2^-115 against Q at 2^115 (scores of ordinary size), and V at 2^-112: the tolerance of
+    ordinary values, the scores' dominated by their own rounding."""
+    g = torch.Generator().manual_seed(L)
+    qkv = _rand(g, S * L, 3 * heads * 64)
+    q, k, v = qkv.view(S * L, 3, heads, 64).unbind(1)
+    if which == "k":
+        q.mul_(2.0 ** 115)
+        k.mul_(2.0 ** -115)
+    else:
+        v.mul_(2.0 ** -112)
+    out, ref = _attention(ctx, qkv, S, L, heads), _attention_ref(qkv, S, L, heads)
+    err = float((out - ref).norm() / ref.norm())
+    report("f32.attention.tiny", L=L, which=which, err=f"{err:.2e}")
     assert err <= 2.0 ** -24 * ((6 * max(L, 16) / 16) ** 0.5 + 64)
 
 
