@@ -898,7 +898,6 @@ template <typename T, int BM, int BN, int WM, int WN, int STAGES, int BK, int AM
 __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const GemmArgs p, int tiles_m, int tiles_n) {
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32, NW = WM * WN;
   constexpr int ES = sizeof(T), KE = 16 / ES;  // bytes per element, elements per 16-byte chunk
-  constexpr int MPI = ES == 4 ? 6 : 1;         // MFMA instructions per tile pair and k-step
   // A tile row holds BK elements = RB bytes = CPR 16-byte chunks; one load instruction of a
   // wave fills RPI rows (1 KiB). Chunk c of row r sits in slot c ^ ((r >> SH) & (CPR - 1)), which
   // keeps the 16 lanes of every ds_read_b128 phase on distinct banks.
@@ -1294,7 +1293,7 @@ __global__ void __launch_bounds__(WM * WN * 64, MINB) gemm_mfma_kernel(const Gem
             // interleave the LDS reads with this step's MFMAs
 #pragma unroll
             for (int k = 0; k < NF; ++k) {
-              __builtin_amdgcn_sched_group_barrier(0x008, MM * MPI / NF > 0 ? MM * MPI / NF : 1, 0);
+              __builtin_amdgcn_sched_group_barrier(0x008, MM / NF > 0 ? MM / NF : 1, 0);
               __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
           }
@@ -1498,6 +1497,8 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
     b.ldp = (a.N + 7) / 8 * 8;
     b.kper = cdiv(cdiv(a.K, BK), S);
   }
+  constexpr bool SPLITS = sizeof(T) == 2 || BM != 128 || BN != 64;  // fp32 128x64 tiles never split (f32_plan)
+  SPLAT_CHECK(SPLITS || S == 1, BAD_ARGUMENT, "gemm: no split-K on this tile");
   dim3 grid(tm * tn * S);
 #define SPLAT_GO(AM, RL, EP) \
   hipLaunchKernelGGL((gemm_mfma_kernel<T, BM, BN, WM, WN, STAGES, BK, AM, RL, EP, MINB, AR>), grid, dim3(WM * WN * 64), 0, ex.stream, \
@@ -1514,8 +1515,9 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
     else SPLAT_CHECK(false, BAD_ARGUMENT, "gemm: fused head needs a bf16 128-column tile");
   } else if (a.amode == A_ROWS) {
     if constexpr (!TAP_ONLY) {
-      if (epi == EPI_PART) SPLAT_GO(A_ROWS, false, EPI_PART);
-      else if (epi == EPI_BIAS) SPLAT_GO(A_ROWS, false, EPI_BIAS);
+      if (epi == EPI_PART) {
+        if constexpr (SPLITS) SPLAT_GO(A_ROWS, false, EPI_PART);
+      } else if (epi == EPI_BIAS) SPLAT_GO(A_ROWS, false, EPI_BIAS);
       else if (epi == EPI_RES) SPLAT_GO(A_ROWS, false, EPI_RES);
       else if (epi == EPI_LN) SPLAT_GO(A_ROWS, false, EPI_LN);
       else if (epi == EPI_RESLN) SPLAT_GO(A_ROWS, false, EPI_RESLN);
@@ -1523,8 +1525,10 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
     }
   } else if (tap) {
     if (epi == EPI_PART) {
-      if (a.relu_in) SPLAT_GO(A_CONV_TAP, true, EPI_PART);
-      else SPLAT_GO(A_CONV_TAP, false, EPI_PART);
+      if constexpr (SPLITS) {
+        if (a.relu_in) SPLAT_GO(A_CONV_TAP, true, EPI_PART);
+        else SPLAT_GO(A_CONV_TAP, false, EPI_PART);
+      }
     } else if (epi == EPI_BIAS) {
       if (a.relu_in) SPLAT_GO(A_CONV_TAP, true, EPI_BIAS);
       else SPLAT_GO(A_CONV_TAP, false, EPI_BIAS);
@@ -1536,8 +1540,9 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
     }
   } else {
     if constexpr (!TAP_ONLY) {
-      if (epi == EPI_PART) SPLAT_GO(A_CONV, false, EPI_PART);
-      else if (epi == EPI_BIAS) SPLAT_GO(A_CONV, false, EPI_BIAS);
+      if (epi == EPI_PART) {
+        if constexpr (SPLITS) SPLAT_GO(A_CONV, false, EPI_PART);
+      } else if (epi == EPI_BIAS) SPLAT_GO(A_CONV, false, EPI_BIAS);
       else SPLAT_GO(A_CONV, false, EPI_FULL);
     }
   }
@@ -1571,7 +1576,7 @@ static BfShape bf_shape(BfCfg c) {
     case CFG_F128x128: return {128, 128, 2};
     case CFG_F64x64: return {64, 64, 4};
     case CFG_192x128D: return {192, 128, 2};
-    case CFG_F128x64: return {128, 64, 3};
+    case CFG_F128x64: return {128, 64, 2};
     default: return {128, 128, 1};
   }
 }
@@ -1624,27 +1629,15 @@ static BfShape bf_shape(BfCfg c) {
 // spans at least 16 k-tiles is cut into S >= 2 slices of at least 8 k-tiles, S * tiles within
 // one round. The slices write fp32 partials; a second kernel sums them and applies the
 // epilogue (the DPT head's coarse-level convs: M = 1596, K = 6912, 14 tiles of 256x128).
-// fp32 (64x64 tiles): at most 160 tiles, one round of slices of at least 6 k-tiles or two rounds of at
-// least 12 (us unsplit / split, the reduce included: 1297x384x1536 126 tiles 31.6 / 22.4 in 4; 3x3 of 64
-// channels, K = 576: 81 tiles 16.8 / 14.2 in 3, 21 tiles 16.2 / 12.1 in 3; 324 tiles lose, 26.2 / 29.7).
-// The two larger fp32 tiles never split: they are taken where 64x64 tiles already fill the chip (162 tiles
-// of 128x64, K = 576: 32.9 in 2 with the reduce, 23.5 as 324 tiles of 64x64 unsplit).
+// (The wider fp32 tiles: f32_plan.)
 static int split_factor(const GemmArgs& a, BfCfg c) {
   if (a.hw3 || a.ln_in) return 1;  // the fused head needs whole tiles, a folded LayerNorm whole rows of K
   const BfShape sh = bf_shape(c);
   const long tiles = long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn);
   const long slots = long(GEMM_CUS) * sh.per_cu;
   const int nk = cdiv(a.K, a.dt == F32 ? 32 : 64);
-  if (c == CFG_F128x128 || c == CFG_F128x64) return 1;
-  int S;
-  if (c == CFG_F64x64) {
-    if (tiles > 160) return 1;
-    S = int(std::max(std::min<long>(nk / 6, GEMM_CUS / tiles), std::min<long>(nk / 12, 2 * GEMM_CUS / tiles)));
-    S = std::min(S, 16);
-  } else {
-    if (2 * tiles > slots || nk < 16) return 1;
-    S = int(std::min<long>(nk / 8, slots / tiles));
-  }
+  if (2 * tiles > slots || nk < 16) return 1;
+  const int S = int(std::min<long>(nk / 8, slots / tiles));
   if (S < 2) return 1;
   return cdiv(nk, cdiv(nk, S));  // every slice non-empty
 }
@@ -1652,37 +1645,64 @@ static size_t split_bytes(const GemmArgs& a, int S) {
   return S > 1 ? size_t(S) * a.M * ((a.N + 7) / 8 * 8) * sizeof(float) : 0;
 }
 
-// fp32: six matrix products of split parts a k-step, and 44 VALU instructions for every 8 values
-// a wave splits, so a wave's share of the tile sets the ratio of the two: 64x64 (128x128 tiles)
-// is bound by the matrix cores, 32x32 (64x64 tiles) by the VALU. Cost of a choice: the tiles of
-// the fullest CU times area / eff, and a wave alone on its SIMD overlaps less except in the 64x64
-// shape. Measured (bias epilogue, us for 128x128 / 128x64 / 64x64): 5838x1152x384 37 / 45 / 50,
-// 5838x384x1536 58 / 74 / 72, 1297x1152x384 20 / 16 / 17, 1297x384x384 18 / 14 / 10, 8192x2048x2048
-// 354 / 432 / 506; 3x3 of 64 channels on 93312 pixels 56 on 128x64, 65 on 64x64.
-// A launch that 64x64 tiles would leave under half full and K allows keeps them and splits K.
-[[maybe_unused]] static BfCfg pick_f32(const GemmArgs& a) {
-  if (a.N <= 32 && !a.qk_dim) return CFG_128x32;
-  if (split_factor(a, CFG_F64x64) > 1) return CFG_F64x64;
-  const BfCfg cands[] = {CFG_F128x128, CFG_F128x64, CFG_F64x64};
-  const double eff[] = {1.0, 0.82, 0.69}, alone[] = {1.0, 1.2, 1.15};
+// fp32: six matrix products of split parts a k-step, and 46 VALU instructions for every 8 values a wave
+// splits, so a wave's share of the tile sets the ratio of the two: 64x64 (128x128 tiles) is bound by the
+// matrix cores, 32x32 (64x64 tiles) by the VALU. The plan, a tile and a number of K slices (not for
+// 128x64), is the cheapest by a model of the time in us: start + tile * n + (32-element k-tiles of a
+// slice) * step, n the blocks of the fullest CU, step with one block a CU (the chip full: more, in
+// proportion to its fill), n steps of `steps` with several; slices add a reduce, 4.5 us and 0.16 a MB
+// of partials. Constants fitted to 106 shapes, every tile, 1 to 8 slices: the choices' geometric mean
+// is the measured best's, 25.8 us.
+// Measured, us (64x64 / 128x64 / 128x128, "in S" with the reduce): 1297x384x384 10.1 (12.0 in 2) / 14.5 /
+// 18.3; 1297x384x1536 30.0 (22.4 in 2, 21.9 in 4) / 46 / 58.7; 1297x1152x384 15.8 / 15.7 / 19.1;
+// 3892x384x1536 50.1 (45.8 in 2) / 47.6 / 59.6 (41.9 in 2); 5838x1152x384 49.5 / 47.7 / 36.2; 5838x384x1536
+// 72.4 / 77.2 / 61.1 (53.5 in 3); 3x3 of 64 channels, 23328 pixels 24.1 / 26.0, 5184 pixels 17.0 (14.3 in
+// 3); 2x2 transposed convolution of 96 channels on 6 x 27x36 11.2 / 13.3 / 15.4.
+struct F32Plan { BfCfg cfg; int S; };
+struct F32Cost {
+  BfCfg cfg;
+  int max_slices;
+  double start, tile, step, fill, steps;  // rows, the row epilogues
+  double start_conv, step_conv, steps_conv;
+  double start_full, tile_full, tile_scalar;  // EPI_FULL: with and without 8-column runs
+};
+[[maybe_unused]] static F32Plan f32_plan(const GemmArgs& a) {
+  if (a.N <= 32 && !a.qk_dim) return {CFG_128x32, split_factor(a, CFG_128x32)};
+  static const F32Cost tiles[] = {{CFG_F64x64, 16, 2.8, 0.7, 0.53, 0.05, 0.50, 4.5, 0.65, 0.51, 3.7, 1.2, 3.0},
+                                  {CFG_F128x64, 1, 2.3, 1.9, 0.83, 0.13, 0.80, 5.2, 0.955, 0.87, 3.8, 3.9, 8.0},
+                                  {CFG_F128x128, 8, 1.6, 3.8, 1.05, 0.30, 1.10, 4.1, 1.22, 1.15, 4.1, 6.0, 24.0}};
+  const bool conv = a.amode != A_ROWS, full = epi_kind(a) == EPI_FULL;
+  const int nk = cdiv(a.K, 32);
   double best = 1e30;
-  BfCfg pick = CFG_F128x128;
-  for (int i = 0; i < 3; ++i) {
-    const BfShape sh = bf_shape(cands[i]);
+  F32Plan plan = {CFG_F64x64, 1};
+  for (const F32Cost& c : tiles) {
+    const BfShape sh = bf_shape(c.cfg);
     if (a.N <= 64 && sh.bn > 64) continue;
-    const long per = (long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn) + GEMM_CUS - 1) / GEMM_CUS;
-    const double cost = double(per) * sh.bm * sh.bn / eff[i] * (per == 1 ? alone[i] : 1.0);
-    if (cost < best * 0.999) { best = cost; pick = cands[i]; }
+    const long tiles_mn = long(cdiv(a.M, sh.bm)) * cdiv(a.N, sh.bn);
+    const double step = conv ? c.step_conv : c.step, steps = conv ? c.steps_conv : c.steps;
+    // a folded LayerNorm takes whole rows of K; more than four blocks a CU leave nothing to fill
+    const int max_s = a.ln_in ? 1 : int(std::max<long>(1, std::min<long>({c.max_slices, nk / 2, 4 * GEMM_CUS / tiles_mn})));
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (s > max_s) break;
+      const int kper = cdiv(nk, s), S = cdiv(nk, kper);  // every slice non-empty
+      if (S != s) continue;
+      const long blocks = tiles_mn * S, n = (blocks + GEMM_CUS - 1) / GEMM_CUS;
+      const bool f = full && S == 1;
+      double t = (f ? c.start_full : conv ? c.start_conv : c.start) + double(n) * (!f ? c.tile : a.epi_vec ? c.tile_full : c.tile_scalar);
+      t += kper * (n == 1 ? step + c.fill * std::min(1.0, double(blocks) / GEMM_CUS) : double(n) * steps);
+      // (the reduce without 8-column runs: 588 x 588 on 6216 pixels 67 us in 2 slices, 55 whole)
+      if (S > 1) t = 1.03 * (t + 4.5 + (0.16e-6 * 4.0 * S + (a.epi_vec ? 0.0 : 4e-6)) * a.M * double(a.N));
+      if (t < best * 0.999) { best = t; plan = {c.cfg, S}; }
+    }
   }
-  return pick;
+  return plan;
 }
 
 template <typename T>
 static bool launch_f32_auto(const Exec& ex, const GemmArgs& a) {
-  const BfCfg c = pick_f32(a);
-  int S = split_factor(a, c);
-  if (S > 1 && !(ex.ws && ex.ws->ptr && ex.ws->cap >= split_bytes(a, S))) S = 1;
-  switch (c) {
+  const F32Plan plan = f32_plan(a);
+  const int S = plan.S > 1 && !(ex.ws && ex.ws->ptr && ex.ws->cap >= split_bytes(a, plan.S)) ? 1 : plan.S;
+  switch (plan.cfg) {
     case CFG_128x32: return launch_mfma<T, 128, 32, 4, 1, 2>(ex, a, S);
     // two blocks a CU enforced: left alone, the everything-else epilogue (EPI_FULL) took 64 registers
     // more, one block (us, one block -> two: 3x3 of 128 channels with ReLU on load and residual on 93312
@@ -2044,7 +2064,7 @@ void gemm(const Exec& ex, const GemmArgs& args) {
                     (reinterpret_cast<uintptr_t>(a.ln_copy) & 15) == 0,
                 BAD_ARGUMENT, "gemm: row statistics need fp32 rows and N a multiple of the group");
   if (ex.dry && ex.ws && a.M > 0 && mfma_path_ok(a))  // size the split-K partials of the real run
-    ex.ws->need = std::max(ex.ws->need, split_bytes(a, split_factor(a, a.dt == F32 ? pick_f32(a) : pick_bf16(a))));
+    ex.ws->need = std::max(ex.ws->need, split_bytes(a, a.dt == F32 ? f32_plan(a).S : split_factor(a, pick_bf16(a))));
   if (ex.dry || a.M == 0) return;
   const double es = a.dt == F32 ? 4 : 2, mn = double(a.M) * a.N;
   const double abytes = a.amode == A_ROWS ? double(a.M) * a.K * es : double(a.V) * a.Hi * a.Wi * a.Cin * es;

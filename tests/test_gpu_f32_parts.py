@@ -39,12 +39,42 @@ def _gemm(ctx, A, W, bias):
     return out
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (1, 8, 4), (31, 32, 32), (33, 24, 68), (64, 64, 96), (65, 72, 36),        # 128x32 and 64x64 tiles, K tails
-    (1297, 384, 384), (1297, 1152, 384), (200, 64, 1536), (65, 64, 3456),     # 64x64, 128x64; K split
-    (2100, 1152, 64), (5838, 384, 100), (4097, 512, 128),                     # 128x128, ragged last tiles
+def f32_plan(M, N, K, conv=False, ln=False):
+    """csrc/gemm.hip f32_plan for N > 32, 8-column runs and the row epilogues: (rows, columns of the tile, K slices)."""
+    tiles = [(64, 64, 16, 2.8, 0.7, 0.53, 0.05, 0.50, 4.5, 0.65, 0.51),
+             (128, 64, 1, 2.3, 1.9, 0.83, 0.13, 0.80, 5.2, 0.955, 0.87),
+             (128, 128, 8, 1.6, 3.8, 1.05, 0.30, 1.10, 4.1, 1.22, 1.15)]
+    nk, best, plan = -(-K // 32), 1e30, None
+    for bm, bn, cap, start, tile, step, fill, steps, cstart, cstep, csteps in tiles:
+        if N <= 64 and bn > 64:
+            continue
+        if conv:
+            start, step, steps = cstart, cstep, csteps
+        mn = -(-M // bm) * -(-N // bn)
+        cap = 1 if ln else max(1, min(cap, nk // 2, 1024 // mn))
+        for s in (1, 2, 3, 4, 6, 8, 12, 16):
+            kper = -(-nk // s)
+            if s > cap or -(-nk // kper) != s:
+                continue
+            n = -(-mn * s // 256)
+            t = start + n * tile + kper * (step + fill * min(1.0, mn * s / 256) if n == 1 else n * steps)
+            if s > 1:
+                t = 1.03 * (t + 4.5 + 0.16e-6 * 4.0 * s * M * N)
+            if t < best * 0.999:
+                best, plan = t, (bm, bn, s)
+    return plan
+
+
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 8, 4, None), (31, 32, 32, None), (33, 24, 68, None),                   # 128x32, K tails
+    (64, 64, 96, (64, 64, 1)), (65, 72, 36, (64, 64, 1)), (1297, 384, 384, (64, 64, 1)),
+    (200, 64, 1536, (64, 64, 16)), (65, 64, 3456, (64, 64, 16)), (1297, 384, 1536, (64, 64, 4)),   # K split
+    (1301, 1096, 384, (128, 64, 1)), (1150, 1152, 420, (128, 64, 1)),          # 128x64, ragged
+    (2100, 1152, 68, (128, 128, 1)), (5188, 1152, 384, (128, 128, 1)), (4097, 1544, 132, (128, 128, 1)),
+    (2000, 3072, 1024, (128, 128, 1)), (3893, 384, 1540, (128, 128, 2)), (1296, 256, 6912, (128, 128, 8)),
 ])
-def test_gemm_matches_float64(ctx, M, N, K):
+def test_gemm_matches_float64(ctx, M, N, K, tile):
+    assert tile is None or f32_plan(M, N, K) == tile
     g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
     A, W, b = _rand(g, M, K), _rand(g, N, K) * K ** -0.5, _rand(g, N)
     out = _gemm(ctx, A, W, b).double()
@@ -52,6 +82,56 @@ def test_gemm_matches_float64(ctx, M, N, K):
     err = float((out - ref).norm() / ref.norm())
     report("f32.gemm", M=M, N=N, K=K, err=f"{err:.2e}", tol=f"{_tol(K):.2e}")
     assert err <= _tol(K)
+
+
+@pytest.mark.parametrize("M,N,act,tile", [(640, 384, 0, (64, 64, 1)), (1297, 1152, 0, (128, 64, 1)),
+                                          (1150, 1536, 2, (128, 64, 1)), (3892, 1536, 2, (128, 128, 1))])
+def test_folded_layer_norm_matches_float64(ctx, M, N, act, tile):
+    """Statistics and the folded-LayerNorm GEMM on each tile. Beside the sum's roundings: the row's mean, variance
+    and their use, the bias and the activation, within eight more of 2^-24."""
+    K = 384
+    assert f32_plan(M, N, K, ln=True) == tile
+    g = torch.Generator().manual_seed(M)
+    x, W, b = _rand(g, M, K) + 0.1, _rand(g, N, K) * K ** -0.5, _rand(g, N)
+    gamma, beta = 1 + 0.1 * _rand(g, K), 0.1 * _rand(g, K)
+    Wf = (W * gamma).contiguous()
+    c1, bf = Wf.double().sum(1).float(), (b.double() + W.double() @ beta.double()).float()
+    stats, out = torch.empty(M, K // 64, 2, device="cuda"), torch.empty(M, N, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_ln_stats(x.data_ptr(), M, K, 64, stats.data_ptr(), splathip.F32)
+    ctx.kernel_gemm_ln(splathip.F32, x.data_ptr(), M, K, Wf.data_ptr(), N, K, bf.data_ptr(), act, out.data_ptr(), True,
+                       ln_in=stats.data_ptr(), c1=c1.data_ptr(), eps=1e-6)
+    ctx.synchronize()
+    ref = torch.nn.functional.layer_norm(x.double(), (K,), None, None, 1e-6) @ Wf.double().t() + bf.double()
+    if act == 2:
+        ref = torch.nn.functional.gelu(ref)
+    err = float((out.double() - ref).norm() / ref.norm())
+    report("f32.gemm_ln", M=M, N=N, act=act, err=f"{err:.2e}")
+    assert err <= 2.0 ** -24 * ((6 * K / 16) ** 0.5 + 8)
+
+
+@pytest.mark.parametrize("M,K,tile", [(1297, 384, (64, 64, 1)), (3892, 384, (128, 64, 1)), (5838, 384, (128, 128, 1)),
+                                      (1297, 1536, (64, 64, 4)), (3892, 1536, (128, 128, 2))])
+def test_residual_statistics_match_float64(ctx, M, K, tile):
+    """out = res + gamma (A W^T + b) and its row statistics on each tile, whole and split: the sum's roundings and
+    three of the epilogue; a group's sums take 64 more."""
+    N = 384
+    assert f32_plan(M, N, K) == tile
+    g = torch.Generator().manual_seed(M + K)
+    A, W, b, gam, res = _rand(g, M, K), _rand(g, N, K) * K ** -0.5, _rand(g, N), _rand(g, N), _rand(g, M, N)
+    out, stats = torch.empty(M, N, device="cuda"), torch.empty(M, N // 64, 2, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_gemm_ln(splathip.F32, A.data_ptr(), M, K, W.data_ptr(), N, K, b.data_ptr(), 0, out.data_ptr(), True,
+                       gamma=gam.data_ptr(), res=res.data_ptr(), ln_out=stats.data_ptr(), group=64)
+    ctx.synchronize()
+    ref = res.double() + gam.double() * (A.double() @ W.double().t() + b.double())
+    err = float((out.double() - ref).norm() / ref.norm())
+    o = out.double().view(M, N // 64, 64)
+    want = torch.stack([o.sum(-1), (o * o).sum(-1)], -1)
+    serr = ((stats.double() - want).abs() / torch.stack([o.abs().sum(-1), (o * o).sum(-1)], -1)).max()
+    report("f32.gemm_res", M=M, K=K, err=f"{err:.2e}", stats=f"{float(serr):.2e}")
+    assert err <= 2.0 ** -24 * ((6 * K / 16) ** 0.5 + 3)
+    assert float(serr) <= 64 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("exp", [-55, 40])
@@ -109,8 +189,9 @@ def _same(out, ref, tol):
     assert err <= tol, err
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 96, 64), (140, 64, 1536), (2100, 1152, 64)])  # 64x64 / 128x64, split, 128x128
+@pytest.mark.parametrize("M,N,K", [(70, 96, 64), (140, 64, 1536), (1297, 1152, 384), (2100, 1152, 64)])
 def test_gemm_special_values(ctx, M, N, K):
+    """64x64 tiles, whole and split, 128x64 and 128x128."""
     g = torch.Generator().manual_seed(9)
     A, W = _rand(g, M, K), _rand(g, N, K)
     A[3, 5], A[40, 7], A[41, K - 1] = float("inf"), float("nan"), float("-inf")
