@@ -221,6 +221,7 @@ __device__ inline Split8 split8(const float (&x)[8], uint32_t& lost) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       o[q][i] = pack_bf16x2(a, b);
+      asm("" : "+v"(o[q][i]));  // one conversion: the compiler would make another for the halves below
       a -= __uint_as_float(o[q][i] << 16);
       b -= __uint_as_float(o[q][i] & 0xffff0000u);
     }

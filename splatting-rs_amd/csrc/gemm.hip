@@ -1650,14 +1650,14 @@ static size_t split_bytes(const GemmArgs& a, int S) {
 // matrix cores, 32x32 (64x64 tiles) by the VALU. The plan, a tile and a number of K slices (not for
 // 128x64), is the cheapest by a model of the time in us: start + tile * n + (32-element k-tiles of a
 // slice) * step, n the blocks of the fullest CU, step with one block a CU (the chip full: more, in
-// proportion to its fill), n steps of `steps` with several; slices add a reduce, 4.5 us and 0.16 a MB
-// of partials. Constants fitted to 106 shapes, every tile, 1 to 8 slices: the choices' geometric mean
-// is the measured best's, 25.8 us.
-// Measured, us (64x64 / 128x64 / 128x128, "in S" with the reduce): 1297x384x384 10.1 (12.0 in 2) / 14.5 /
-// 18.3; 1297x384x1536 30.0 (22.4 in 2, 21.9 in 4) / 46 / 58.7; 1297x1152x384 15.8 / 15.7 / 19.1;
-// 3892x384x1536 50.1 (45.8 in 2) / 47.6 / 59.6 (41.9 in 2); 5838x1152x384 49.5 / 47.7 / 36.2; 5838x384x1536
-// 72.4 / 77.2 / 61.1 (53.5 in 3); 3x3 of 64 channels, 23328 pixels 24.1 / 26.0, 5184 pixels 17.0 (14.3 in
-// 3); 2x2 transposed convolution of 96 channels on 6 x 27x36 11.2 / 13.3 / 15.4.
+// proportion to its fill), n steps of `steps` with several; slices add a reduce, 4.3 us and 0.16 a MB
+// of partials. Constants fitted to 103 shapes, every tile, 1 to 16 slices: the choices' geometric mean is
+// 25.0 us, the measured best's 24.8.
+// Measured, us (64x64 / 128x64 / 128x128, "in S" with the reduce): 1297x384x384 9.6 (11.9 in 2) / 13.9 /
+// 17.5; 1297x384x1536 28.3 (21.3 in 2, 21.8 in 4) / 43.8 / 55.7; 1297x1152x384 14.6 / 15.4 / 18.4;
+// 3892x384x1536 45.6 (43.4 in 2) / 46.7 / 56.7 (40.4 in 2); 5838x1152x384 45.5 / 44.3 / 35.0; 5838x384x1536
+// 67.5 / 74.2 / 58.3 (52.1 in 3); 3x3 of 64 channels, 23328 pixels 22.7 / 24.9, 5184 pixels 16.1 (13.9 in
+// 3); 2x2 transposed convolution of 96 channels on 6 x 27x36 10.9 / 12.8 / 15.0.
 struct F32Plan { BfCfg cfg; int S; };
 struct F32Cost {
   BfCfg cfg;
@@ -1668,9 +1668,9 @@ struct F32Cost {
 };
 [[maybe_unused]] static F32Plan f32_plan(const GemmArgs& a) {
   if (a.N <= 32 && !a.qk_dim) return {CFG_128x32, split_factor(a, CFG_128x32)};
-  static const F32Cost tiles[] = {{CFG_F64x64, 16, 2.8, 0.7, 0.53, 0.05, 0.50, 4.5, 0.65, 0.51, 3.7, 1.2, 3.0},
-                                  {CFG_F128x64, 1, 2.3, 1.9, 0.83, 0.13, 0.80, 5.2, 0.955, 0.87, 3.8, 3.9, 8.0},
-                                  {CFG_F128x128, 8, 1.6, 3.8, 1.05, 0.30, 1.10, 4.1, 1.22, 1.15, 4.1, 6.0, 24.0}};
+  static const F32Cost tiles[] = {{CFG_F64x64, 16, 2.9, 0.45, 0.49, 0.07, 0.47, 4.7, 0.61, 0.53, 3.5, 1.1, 3.0},
+                                  {CFG_F128x64, 1, 1.9, 1.9, 0.785, 0.20, 0.75, 5.6, 0.90, 0.83, 3.9, 3.9, 8.0},
+                                  {CFG_F128x128, 8, 1.4, 3.9, 0.985, 0.31, 1.05, 4.2, 1.17, 1.10, 3.9, 6.0, 24.0}};
   const bool conv = a.amode != A_ROWS, full = epi_kind(a) == EPI_FULL;
   const int nk = cdiv(a.K, 32);
   double best = 1e30;
@@ -1691,7 +1691,7 @@ struct F32Cost {
       double t = (f ? c.start_full : conv ? c.start_conv : c.start) + double(n) * (!f ? c.tile : a.epi_vec ? c.tile_full : c.tile_scalar);
       t += kper * (n == 1 ? step + c.fill * std::min(1.0, double(blocks) / GEMM_CUS) : double(n) * steps);
       // (the reduce without 8-column runs: 588 x 588 on 6216 pixels 67 us in 2 slices, 55 whole)
-      if (S > 1) t = 1.03 * (t + 4.5 + (0.16e-6 * 4.0 * S + (a.epi_vec ? 0.0 : 4e-6)) * a.M * double(a.N));
+      if (S > 1) t = 1.02 * (t + 4.3 + (0.16e-6 * 4.0 * S + (a.epi_vec ? 0.0 : 4e-6)) * a.M * double(a.N));
       if (t < best * 0.999) { best = t; plan = {c.cfg, S}; }
     }
   }

@@ -41,9 +41,9 @@ def _gemm(ctx, A, W, bias):
 
 def f32_plan(M, N, K, conv=False, ln=False):
     """csrc/gemm.hip f32_plan for N > 32, 8-column runs and the row epilogues: (rows, columns of the tile, K slices)."""
-    tiles = [(64, 64, 16, 2.8, 0.7, 0.53, 0.05, 0.50, 4.5, 0.65, 0.51),
-             (128, 64, 1, 2.3, 1.9, 0.83, 0.13, 0.80, 5.2, 0.955, 0.87),
-             (128, 128, 8, 1.6, 3.8, 1.05, 0.30, 1.10, 4.1, 1.22, 1.15)]
+    tiles = [(64, 64, 16, 2.9, 0.45, 0.49, 0.07, 0.47, 4.7, 0.61, 0.53),
+             (128, 64, 1, 1.9, 1.9, 0.785, 0.20, 0.75, 5.6, 0.90, 0.83),
+             (128, 128, 8, 1.4, 3.9, 0.985, 0.31, 1.05, 4.2, 1.17, 1.10)]
     nk, best, plan = -(-K // 32), 1e30, None
     for bm, bn, cap, start, tile, step, fill, steps, cstart, cstep, csteps in tiles:
         if N <= 64 and bn > 64:
@@ -59,7 +59,7 @@ def f32_plan(M, N, K, conv=False, ln=False):
             n = -(-mn * s // 256)
             t = start + n * tile + kper * (step + fill * min(1.0, mn * s / 256) if n == 1 else n * steps)
             if s > 1:
-                t = 1.03 * (t + 4.5 + 0.16e-6 * 4.0 * s * M * N)
+                t = 1.02 * (t + 4.3 + 0.16e-6 * 4.0 * s * M * N)
             if t < best * 0.999:
                 best, plan = t, (bm, bn, s)
     return plan
@@ -69,9 +69,9 @@ def f32_plan(M, N, K, conv=False, ln=False):
     (1, 8, 4, None), (31, 32, 32, None), (33, 24, 68, None),                   # 128x32, K tails
     (64, 64, 96, (64, 64, 1)), (65, 72, 36, (64, 64, 1)), (1297, 384, 384, (64, 64, 1)),
     (200, 64, 1536, (64, 64, 16)), (65, 64, 3456, (64, 64, 16)), (1297, 384, 1536, (64, 64, 4)),   # K split
-    (1301, 1096, 384, (128, 64, 1)), (1150, 1152, 420, (128, 64, 1)),          # 128x64, ragged
-    (2100, 1152, 68, (128, 128, 1)), (5188, 1152, 384, (128, 128, 1)), (4097, 1544, 132, (128, 128, 1)),
-    (2000, 3072, 1024, (128, 128, 1)), (3893, 384, 1540, (128, 128, 2)), (1296, 256, 6912, (128, 128, 8)),
+    (1200, 1096, 384, (128, 64, 1)), (1150, 1152, 420, (128, 64, 1)), (3893, 384, 388, (128, 64, 1)),   # 128x64, ragged
+    (2100, 1152, 68, (64, 64, 1)), (5188, 1152, 384, (128, 128, 1)), (4097, 1544, 132, (128, 128, 1)),
+    (2000, 3072, 1024, (128, 128, 1)), (3893, 384, 1540, (128, 128, 2)), (1296, 256, 6912, (64, 64, 6)),
 ])
 def test_gemm_matches_float64(ctx, M, N, K, tile):
     assert tile is None or f32_plan(M, N, K) == tile
@@ -84,8 +84,8 @@ def test_gemm_matches_float64(ctx, M, N, K, tile):
     assert err <= _tol(K)
 
 
-@pytest.mark.parametrize("M,N,act,tile", [(640, 384, 0, (64, 64, 1)), (1297, 1152, 0, (128, 64, 1)),
-                                          (1150, 1536, 2, (128, 64, 1)), (3892, 1536, 2, (128, 128, 1))])
+@pytest.mark.parametrize("M,N,act,tile", [(640, 384, 0, (64, 64, 1)), (1200, 1152, 0, (128, 64, 1)),
+                                          (1000, 1536, 2, (128, 64, 1)), (3892, 1536, 2, (128, 128, 1))])
 def test_folded_layer_norm_matches_float64(ctx, M, N, act, tile):
     """Statistics and the folded-LayerNorm GEMM on each tile. Beside the sum's roundings: the row's mean, variance
     and their use, the bias and the activation, within eight more of 2^-24."""
@@ -134,6 +134,25 @@ def test_residual_statistics_match_float64(ctx, M, K, tile):
     assert float(serr) <= 64 * 2.0 ** -24
 
 
+def test_qkv_epilogue_on_128x64_tiles(ctx, tmp_path):
+    """DA3-Small on 2 views of 21x28 patches: the cross-view blocks' qkv (1178 rows) runs the folded LayerNorm
+    with qk-norm and RoPE on 128x64 tiles. Against the CPU oracle, both in fp32."""
+    from oracle import da3 as OD
+    from splathip import specs, synth
+    assert f32_plan(2 * (21 * 28 + 1), 1152, 384, ln=True) == (128, 64, 1)
+    spec = specs.DA3_VARIANTS["small"]
+    w = synth.generate(synth.da3_shapes(spec), seed=1, layer_scale=1.0)
+    path = str(tmp_path / "da3.safetensors")
+    synth.save(path, w)
+    images = synth.procedural_images(2, 294, 392, seed=2)
+    ctx.load_da3(path, "small", "f32")
+    out, ref = ctx.da3_forward_raw(images), OD.forward_raw(w, spec, images)
+    want = ref["depth"].numpy()
+    err = float(np.max(np.abs(out["depth"] - want) / want))
+    report("f32.da3", err=f"{err:.2e}")
+    assert err < 1e-4
+
+
 @pytest.mark.parametrize("exp", [-55, 40])
 def test_gemm_wide_range(ctx, exp):
     """Rows and columns spread over 2^+-20 around 2^exp: every row is right by itself."""
@@ -147,7 +166,7 @@ def test_gemm_wide_range(ctx, exp):
     assert err <= _tol(256)
 
 
-@pytest.mark.parametrize("M,N,K", [(130, 96, 256), (140, 64, 1536), (70, 96, 128), (2100, 1152, 64)])
+@pytest.mark.parametrize("M,N,K", [(130, 96, 256), (140, 64, 1536), (1200, 1152, 68), (4097, 1544, 132)])
 @pytest.mark.parametrize("side", ["a", "w"])
 def test_gemm_tiny_values(ctx, M, N, K, side):
     """One operand's rows (of A, or of W) lie at 2^-126 to 2^-90, where the third part of a split falls under
@@ -189,9 +208,10 @@ def _same(out, ref, tol):
     assert err <= tol, err
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 96, 64), (140, 64, 1536), (1297, 1152, 384), (2100, 1152, 64)])
+@pytest.mark.parametrize("M,N,K", [(70, 96, 64), (140, 64, 1536), (1200, 1152, 384), (4097, 1544, 132)])
 def test_gemm_special_values(ctx, M, N, K):
     """64x64 tiles, whole and split, 128x64 and 128x128."""
+    assert f32_plan(M, N, K)[:2] == ((64, 64) if M < 200 else (128, 64) if M == 1200 else (128, 128))
     g = torch.Generator().manual_seed(9)
     A, W = _rand(g, M, K), _rand(g, N, K)
     A[3, 5], A[40, 7], A[41, K - 1] = float("inf"), float("nan"), float("-inf")
