@@ -19,6 +19,11 @@
 
 namespace splat {
 
+// This file is compiled twice: with SPLAT_ATTN_F32 only attn_f32_kernel, whose checks rely on infinities
+// and NaN, without it everything else, which the build lets take them for absent.
+void launch_attn_f32(const Exec& ex, const AttnArgs& b, float c);
+
+#ifndef SPLAT_ATTN_F32
 // Device-resident scratch for the key-slice partials of attention launches that must not
 // allocate (splat_kernel_attention_noalloc): one copy per GPU, held until the process ends.
 // Host code never passes `scratch` itself to a kernel (on the host the name is only a stand-in
@@ -67,6 +72,7 @@ void attention_scratch_ordered(int device, hipStream_t stream, const std::functi
   SPLAT_HIP(hipEventRecord(g_scratch_done[device], stream));
   g_scratch_recorded[device] = true;
 }
+#endif
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -150,6 +156,7 @@ template <> struct AttnOps<float> {
 constexpr int ATTN_WAVES = 4;
 constexpr int ATTN_MAX_SPLITS = 8;  // key slices a launch may use (attn_combine_kernel unrolls over them)
 
+#ifndef SPLAT_ATTN_F32
 // SPLIT: the block covers key tiles [split * tps, (split + 1) * tps) and writes its unnormalised
 // O and (max, sum) to p.part for attn_combine_kernel, as the bf16 kernel below does.
 template <typename T, bool SPLIT>
@@ -335,6 +342,7 @@ __global__ void __launch_bounds__(ATTN_WAVES * 64) attn_kernel(const AttnArgs p,
       }
   }
 }
+#endif
 
 // ---------------------------------------------------------------------------------------
 // bf16 main path. Each wave owns QT*32 queries, so every K and V^T fragment read from LDS
@@ -384,6 +392,7 @@ template <int N> __device__ inline void wait_vm() { asm volatile("s_waitcnt vmcn
 
 }  // namespace
 
+#ifndef SPLAT_ATTN_F32
 // SPLIT: the block covers key tiles [split * tps, (split + 1) * tps) of its sequence and writes
 // its unnormalised O and (reference, sum) to p.part; attn_combine_kernel merges the slices.
 // H: the 16-bit storage type of Q, K, V and O (bf16 or f16).
@@ -745,7 +754,9 @@ __global__ void __launch_bounds__(WAVES * 64, QT == 1 ? 4 : 2) attn_bf16_kernel(
     }
   }
 }
+#endif
 
+#ifdef SPLAT_ATTN_F32
 // ---------------------------------------------------------------------------------------
 // fp32 path. 4 waves x 32 queries, 32-key tiles. The plain pass (max-free, as in the bf16 kernel)
 // runs S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16: every operand is split exactly
@@ -1041,6 +1052,13 @@ __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, floa
           make_float4(o[dt][4 * q4] * inv, o[dt][4 * q4 + 1] * inv, o[dt][4 * q4 + 2] * inv, o[dt][4 * q4 + 3] * inv);
 }
 
+void launch_attn_f32(const Exec& ex, const AttnArgs& b, float c) {
+  const dim3 grid(unsigned(long(cdiv(b.L, 128)) * b.heads * b.seqs * b.nsplit));
+  if (b.nsplit > 1) hipLaunchKernelGGL(attn_f32_kernel<true>, grid, dim3(256), 0, ex.stream, b, c);
+  else hipLaunchKernelGGL(attn_f32_kernel<false>, grid, dim3(256), 0, ex.stream, b, c);
+}
+
+#else
 // Merges the key slices of a split launch: per query and head, M = max of the slices' exponent
 // references m_s (their maxima, or 0 for a plain pass), O = sum_s 2^(m_s - M) O_s /
 // sum_s 2^(m_s - M) l_s. One thread per 8 head channels.
@@ -1238,14 +1256,11 @@ void attention(const Exec& ex, const AttnArgs& a) {
   ProfScope ps(ex, "attention", 4.0 * rows * a.L * 64, 4.0 * rows * 64 * (a.dt == F32 ? 4 : 2));
   const float c = a.q_scaled ? 1.f : ATTN_Q_SCALE;  // Q times 1 is exact, rounded or not
   if (f32_fast) {
-    const dim3 grid(unsigned(long(cdiv(a.L, 128)) * a.heads * a.seqs * b.nsplit));
+    launch_attn_f32(ex, b, c);
     if (b.nsplit > 1) {
-      hipLaunchKernelGGL(attn_f32_kernel<true>, grid, dim3(256), 0, ex.stream, b, c);
       SPLAT_HIP(hipGetLastError());
       const long work = long(a.seqs) * a.L * a.heads * 8;
       hipLaunchKernelGGL(attn_combine_kernel<float>, dim3(unsigned((work + 255) / 256)), dim3(256), 0, ex.stream, b);
-    } else {
-      hipLaunchKernelGGL(attn_f32_kernel<false>, grid, dim3(256), 0, ex.stream, b, c);
     }
   } else if (a.dt == F32) {
     const dim3 grid(unsigned(cdiv(a.L, ATTN_WAVES * 32) * b.nsplit), a.heads, a.seqs);
@@ -1264,5 +1279,6 @@ void attention(const Exec& ex, const AttnArgs& a) {
   }
   SPLAT_HIP(hipGetLastError());
 }
+#endif
 
 }  // namespace splat

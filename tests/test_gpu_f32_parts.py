@@ -308,3 +308,29 @@ def test_attention_special_values(ctx):
     assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
     fine = torch.isfinite(ref)
     assert float(((out[fine] - ref[fine]).abs() / (ref[fine].abs() + 1.0)).max()) < 1e-5
+
+
+@pytest.mark.parametrize("S,L,heads", [(1, 40, 2), (1, 1297, 2)])   # unsplit; key slices
+@pytest.mark.parametrize("which", ["nan_q", "inf_k", "nan_k", "big_k", "big_v", "nan_v"])
+def test_attention_operands_outside_bf16(ctx, S, L, heads, which):
+    """One operand value that bf16 parts cannot hold, in head 0: what float64 gives, NaN and infinities in the
+    same places. big: finite, rounds to infinity in bf16; Q is a power of two there, so that no other
+    check sees it."""
+    g = torch.Generator().manual_seed(L + 1)
+    qkv = _rand(g, S * L, 3 * heads * 64)
+    q, k, v = qkv.view(S * L, 3, heads, 64).unbind(1)
+    if which == "nan_q":
+        q[L // 2, 0, 7] = float("nan")
+    elif which in ("inf_k", "nan_k"):
+        k[L // 3, 0, 9] = float(which[:3])
+    elif which == "big_k":
+        q[:, 0, 9] = torch.where(q[:, 0, 9] > 0, 2.0 ** -124, -2.0 ** -124)
+        k[L // 3, 0, 9] = 3.4e38
+    else:
+        v[L // 3, 0, 9] = 3.4e38 if which == "big_v" else float("nan")
+        k[L // 3, 0] = 0.0   # a weight of at most 1 before the division: the sum stays finite
+    out, ref = _attention(ctx, qkv, S, L, heads), _attention_ref(qkv, S, L, heads)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    fine = ~torch.isnan(ref)
+    scale = ref.abs() + 1.0
+    assert float(((out[fine] - ref[fine]).abs() / scale[fine]).max()) <= 2.0 ** -24 * ((6 * max(L, 16) / 16) ** 0.5 + 64)
