@@ -334,3 +334,45 @@ def test_attention_operands_outside_bf16(ctx, S, L, heads, which):
     fine = ~torch.isnan(ref)
     scale = ref.abs() + 1.0
     assert float(((out[fine] - ref[fine]).abs() / scale[fine]).max()) <= 2.0 ** -24 * ((6 * max(L, 16) / 16) ** 0.5 + 64)
+
+
+@pytest.mark.parametrize("V,H,W,C,N,stride,relu", [
+    (1, 18, 18, 96, 64, 1, 0), (1, 18, 18, 96, 64, 1, 1), (1, 18, 18, 96, 64, 2, 1),   # K in slices
+    (3, 108, 144, 32, 64, 1, 1), (1, 60, 60, 64, 32, 1, 0),                         # whole; 128x32
+    (4, 100, 130, 64, 64, 1, 1), (2, 66, 70, 64, 256, 1, 0), (2, 66, 70, 64, 256, 2, 1),   # 128x64; wider
+    (1, 40, 33, 48, 40, 1, 0), (1, 40, 33, 36, 72, 2, 0), (3, 108, 144, 20, 130, 1, 0),    # per-lane addressing
+])
+def test_conv_special_values(ctx, V, H, W, C, N, stride, relu):
+    """An infinite, a NaN and a 3.4e38 pixel, at a corner and inside: such waves redo their sums with a convolution
+    of their own. Every output within K 2^-24 of the sum of its products' magnitudes (any order of an
+    fp32 sum), the others' NaN and infinities in the same places."""
+    g = torch.Generator().manual_seed(H * W + C)
+    x, w, b = _rand(g, V, H, W, C), _rand(g, N, C, 3, 3) * (9 * C) ** -0.5, _rand(g, N)
+    x[0, 0, 0, 3], x[V - 1, H // 2, W // 3, 1] = float("inf"), float("nan")
+    x[0, H - 1, W - 1, 2] = 3.4e38
+    x[V - 1, 3, 5, 0], x[0, 9, 2, 4] = float("-inf"), -3.4e38
+    w[:, 2] *= 0.01
+    w[:, 4] *= 0.01
+    ldw = (9 * C + 63) // 64 * 64
+    wp = torch.zeros(N, ldw, device="cuda")
+    wp[:, :9 * C] = w.permute(0, 2, 3, 1).reshape(N, -1)
+    Ho, Wo = (H - 1) // stride + 1, (W - 1) // stride + 1
+    out = torch.empty(V, Ho, Wo, N, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_conv2d(splathip.F32, x.data_ptr(), V, H, W, C, wp.data_ptr(), N, ldw, 3, stride, b.data_ptr(), relu, 0, 0,
+                      out.data_ptr())
+    ctx.synchronize()
+    xd = x.cpu().double()
+    xd = torch.where(xd < 0, 0.0, xd) if relu else xd   # keeps NaN
+    cols = torch.nn.functional.unfold(xd.permute(0, 3, 1, 2), 3, padding=1, stride=stride).transpose(1, 2)   # [V, P, 9 C]
+    wd = w.cpu().double().reshape(N, -1).t()
+    ref = (cols @ wd + b.cpu().double()).float().reshape(V, Ho, Wo, N)
+    mag = (cols.abs() @ wd.abs()).reshape(V, Ho, Wo, N) + b.cpu().double().abs()
+    out = out.cpu()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
+    fine = torch.isfinite(ref)
+    assert 0 < int((~fine).sum()) < fine.numel() // 2
+    err = float(((out - ref).double().abs()[fine] / mag[fine]).max())
+    report("f32.conv.special", H=H, W=W, C=C, N=N, stride=stride, relu=relu, err=f"{err:.2e}")
+    assert err <= (9 * C + 2) * 2.0 ** -24
