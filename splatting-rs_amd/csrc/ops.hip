@@ -1319,8 +1319,9 @@ __global__ void __launch_bounds__(256) fit_intrinsics_kernel(const float* pts, i
 // launch instead of three) and walks its pixels; one reciprocal serves a projection's two
 // quotients, the focal lengths' are taken once a camera. A call on 6 views 378x504: 37.5 us as three
 // kernels (cameras 4, points 10, cleaning 27) -> 23.2 us.
+// I numbers the pixels of a view: int, or long where a view and a turn past it reach 2^31 pixels.
 constexpr int CAMS = 64, CAMLD = 18;  // R (9), t (3), 1/fx, 1/fy, cx, cy, mean focal
-template <bool LDSCAM>
+template <bool LDSCAM, typename I>
 __global__ void __launch_bounds__(256) recon_points_kernel(
     int V, int H, int W, int bpv, const float* __restrict__ depth, const float* __restrict__ pts_cam,
     const float* __restrict__ conf, const uint8_t* __restrict__ mask, const uint8_t* __restrict__ fg,
@@ -1353,7 +1354,7 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
     __syncthreads();
   }
   const int i = int(blockIdx.x) / bpv, b = int(blockIdx.x) - i * bpv;  // view, block of the view
-  const int hw = H * W;
+  const I hw = I(H) * W;
   const long base = long(i) * hw;
   double own_[LDSCAM ? 1 : CAMLD];
   const double* own = sc + i * CAMLD;
@@ -1362,9 +1363,9 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
     own = own_;
   }
   const double fW = W - 0.5, fH = H - 0.5;
-  for (int pix = b * 256 + int(threadIdx.x); pix < hw; pix += bpv * 256) {
+  for (I pix = b * 256 + int(threadIdx.x); pix < hw; pix += bpv * 256) {
     const long id = base + pix;
-    const int y = pix / W, x = pix - y * W;
+    const int y = int(pix / W), x = int(pix - I(y) * W);
     double p[3];
     if (depth) {
       const double d = depth[id];
@@ -1400,7 +1401,7 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
         // round(u) in [0, W): u in (-0.5, W - 0.5), and there half away from zero is half up
         if (!(u > -0.5 && w > -0.5 && u < fW && w < fH)) continue;
         const double uf = floor(u), wf = floor(w);
-        const int op = (int(wf) + int(w - wf >= 0.5)) * W + int(uf) + int(u - uf >= 0.5);
+        const I op = I(int(wf) + int(w - wf >= 0.5)) * W + int(uf) + int(u - uf >= 0.5);
         const long oj = long(j) * hw + op;
         const float cf = mask && !mask[oj] ? 0.f : conf[oj];
         const float dj = depth ? depth[oj] : pts_cam[oj * 3 + 2];
@@ -1418,20 +1419,24 @@ void reconstruct_geometry(const Exec& ex, int V, int H, int W, const float* dept
   if (ex.dry || V == 0) return;
   const bool da3 = depth != nullptr;
   SPLAT_CHECK(da3 ? pose_enc != nullptr : (pts_cam && quat && trans && fitted), BAD_ARGUMENT, "geometry inputs");
-  SPLAT_CHECK(double(H) * W < 2147483648.0, BAD_SHAPE, "geometry: a view of 2^31 pixels and more");
   const long px = long(V) * H * W;
   ProfScope ps(ex, "geometry", 0.0, double(px) * (da3 ? 4 : 12) * 2 + double(px) * 4 * (V + 2) + double(px) * 12);
   if (!da3) hipLaunchKernelGGL(fit_intrinsics_kernel, dim3(V), dim3(256), 0, ex.stream, pts_cam, H, W, fitted);
   // up to eight blocks a CU (resident together), each within one view, all with the same number of turns
   const int all = cdiv(long(H) * W, 256), turns = cdiv(long(all) * V, 8 * 256), bpv = cdiv(all, turns);
+  const bool wide = long(H) * W + long(bpv) * 256 >= 2147483648L;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(unsigned(V) * bpv), dim3(256), 0, ex.stream, V, H, W, bpv, depth, pts_cam, conf, mask, fg,
+                       pose_enc, quat, trans, fitted, cam, points, conf_out);
+  };
   if (V <= CAMS) {
-    hipLaunchKernelGGL(recon_points_kernel<true>, dim3(unsigned(V) * bpv), dim3(256), 0, ex.stream, V, H, W, bpv, depth,
-                       pts_cam, conf, mask, fg, pose_enc, quat, trans, fitted, cam, points, conf_out);
+    if (wide) launch(recon_points_kernel<true, long>);
+    else launch(recon_points_kernel<true, int>);
   } else {
     hipLaunchKernelGGL(recon_cameras_kernel, dim3(cdiv(V, 64)), dim3(64), 0, ex.stream, V, H, W, pose_enc, quat, trans,
                        fitted, cam);
-    hipLaunchKernelGGL(recon_points_kernel<false>, dim3(unsigned(V) * bpv), dim3(256), 0, ex.stream, V, H, W, bpv, depth,
-                       pts_cam, conf, mask, fg, pose_enc, quat, trans, fitted, cam, points, conf_out);
+    if (wide) launch(recon_points_kernel<false, long>);
+    else launch(recon_points_kernel<false, int>);
   }
   SPLAT_HIP(hipGetLastError());
 }

@@ -72,3 +72,31 @@ def test_points_over_their_source(ctx):
     got = call(both, both)
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
     assert 0 < int((ref[2] == 0).sum()) < conf.numel()
+
+
+@pytest.mark.parametrize("H,W", [(46340, 46340), (46342, 46341)])   # within a turn of 2^31 pixels, and past it
+def test_largest_view(ctx, H, W):
+    """One view whose pixel numbers pass 32 bits on the last turn, or are longer: every confidence is kept, and
+    the points of the last rows and of a sample of pixels are the unprojected depths."""
+    n = H * W
+    if torch.cuda.mem_get_info()[0] < 28 * n:
+        pytest.skip("needs 60 GB of GPU memory")
+    depth = torch.rand(n, device="cuda").add_(1.0)
+    conf = torch.rand(n, device="cuda").add_(1.0)
+    pose = torch.tensor([[0, 0, 0, 0, 0, 0, 1, 0.9, 1.0]], device="cuda")
+    cams = torch.empty(1, 16, dtype=torch.float64, device="cuda")
+    pts, out = torch.full((n, 3), -7.0, device="cuda"), torch.full((n,), -7.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_reconstruct(1, H, W, depth=depth.data_ptr(), pose_encoding=pose.data_ptr(), conf=conf.data_ptr(),
+                           cameras=cams.data_ptr(), points=pts.data_ptr(), conf_out=out.data_ptr())
+    ctx.synchronize()
+    assert torch.equal(out, conf)
+    fx, fy, cx, cy = (float(v) for v in cams[0, 12:])
+    for idx in (torch.arange(n - 600000, n, device="cuda"),
+                torch.randint(0, n, (600000,), device="cuda", generator=torch.Generator("cuda").manual_seed(1))):
+        d = depth[idx].double()
+        x, y = (idx % W).double(), torch.div(idx, W, rounding_mode="floor").double()
+        want = torch.stack([(x - cx) / fx * d, (y - cy) / fy * d, d], -1)
+        assert float((pts[idx].double() - want).abs().max()) <= 2.0 ** -23 * float(want.abs().max())
+    del depth, conf, pts, out
+    torch.cuda.empty_cache()
