@@ -1319,9 +1319,13 @@ __global__ void __launch_bounds__(256) fit_intrinsics_kernel(const float* pts, i
 // launch instead of three) and walks its pixels; one reciprocal serves a projection's two
 // quotients, the focal lengths' are taken once a camera. A call on 6 views 378x504: 37.5 us as three
 // kernels (cameras 4, points 10, cleaning 27) -> 23.2 us.
+// LAZY: the other view's confidence and mask are read only where the depth passes, one memory latency
+// later. Taken once the maps together exceed the L2s (8 x 4 MB) and traffic counts for more: 24 views
+// 378x504 of rough depths with a foreground, 386 us as three kernels, 440 -> 294; smooth ones 240 -> 255; 6
+// views (10 MB) 22.1 -> 23.8, so not there.
 // I numbers the pixels of a view: int, or long where a view and a turn past it reach 2^31 pixels.
 constexpr int CAMS = 64, CAMLD = 18;  // R (9), t (3), 1/fx, 1/fy, cx, cy, mean focal
-template <bool LDSCAM, typename I>
+template <bool LDSCAM, typename I, bool LAZY>
 __global__ void __launch_bounds__(256) recon_points_kernel(
     int V, int H, int W, int bpv, const float* __restrict__ depth, const float* __restrict__ pts_cam,
     const float* __restrict__ conf, const uint8_t* __restrict__ mask, const uint8_t* __restrict__ fg,
@@ -1403,9 +1407,15 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
         const double uf = floor(u), wf = floor(w);
         const I op = I(int(wf) + int(w - wf >= 0.5)) * W + int(uf) + int(u - uf >= 0.5);
         const long oj = long(j) * hw + op;
-        const float cf = mask && !mask[oj] ? 0.f : conf[oj];
-        const float dj = depth ? depth[oj] : pts_cam[oj * 3 + 2];
-        if ((!fg || fg[oj]) && qz < (1.0 - 0.02) * double(dj) && ci < cf) zero = true;
+        auto conf_j = [&] { return mask && !mask[oj] ? 0.f : conf[oj]; };
+        if constexpr (LAZY) {
+          const float dj = depth ? depth[oj] : pts_cam[oj * 3 + 2];
+          const bool fore = !fg || fg[oj];
+          if (fore && qz < (1.0 - 0.02) * double(dj)) zero = ci < conf_j();
+        } else {
+          const float cf = conf_j(), dj = depth ? depth[oj] : pts_cam[oj * 3 + 2];
+          if ((!fg || fg[oj]) && qz < (1.0 - 0.02) * double(dj) && ci < cf) zero = true;
+        }
       }
     }
     conf_out[id] = zero ? 0.f : ci;
@@ -1429,14 +1439,17 @@ void reconstruct_geometry(const Exec& ex, int V, int H, int W, const float* dept
     hipLaunchKernelGGL(kernel, dim3(unsigned(V) * bpv), dim3(256), 0, ex.stream, V, H, W, bpv, depth, pts_cam, conf, mask, fg,
                        pose_enc, quat, trans, fitted, cam, points, conf_out);
   };
+  const bool lazy = double(px) * ((da3 ? 4 : 12) + 4 + (mask ? 1 : 0) + (fg ? 1 : 0)) > 8.0 * (4 << 20);
   if (V <= CAMS) {
-    if (wide) launch(recon_points_kernel<true, long>);
-    else launch(recon_points_kernel<true, int>);
+    if (wide) launch(recon_points_kernel<true, long, true>);
+    else if (lazy) launch(recon_points_kernel<true, int, true>);
+    else launch(recon_points_kernel<true, int, false>);
   } else {
     hipLaunchKernelGGL(recon_cameras_kernel, dim3(cdiv(V, 64)), dim3(64), 0, ex.stream, V, H, W, pose_enc, quat, trans,
                        fitted, cam);
-    if (wide) launch(recon_points_kernel<false, long>);
-    else launch(recon_points_kernel<false, int>);
+    if (wide) launch(recon_points_kernel<false, long, true>);
+    else if (lazy) launch(recon_points_kernel<false, int, true>);
+    else launch(recon_points_kernel<false, int, false>);
   }
   SPLAT_HIP(hipGetLastError());
 }
