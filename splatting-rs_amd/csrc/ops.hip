@@ -1317,14 +1317,28 @@ __global__ void __launch_bounds__(256) fit_intrinsics_kernel(const float* pts, i
 // Bound by f64 VALU work (V - 1 projections a pixel) and the gathers from L2. A block stays in one
 // view, keeps every camera in LDS (LDSCAM, V <= CAMS: computed by the block's first threads, one
 // launch instead of three) and walks its pixels; one reciprocal serves a projection's two
-// quotients, the focal lengths' are taken once a camera. A call on 6 views 378x504: 37.5 us as three
+// quotients, the focal lengths' are taken once a camera; every quotient is the division's, so a projection
+// half way between two pixels goes where f64::round sends it. A call on 6 views 378x504: 37.5 us as three
 // kernels (cameras 4, points 10, cleaning 27) -> 23.2 us.
 // LAZY: the other view's confidence and mask are read only where the depth passes, one memory latency
 // later. Taken once the maps together exceed the L2s (8 x 4 MB) and traffic counts for more: 24 views
 // 378x504 of rough depths with a foreground, 386 us as three kernels, 440 -> 294; smooth ones 240 -> 255; 6
 // views (10 MB) 22.1 -> 23.8, so not there.
 // I numbers the pixels of a view: int, or long where a view and a turn past it reach 2^31 pixels.
-constexpr int CAMS = 64, CAMLD = 18;  // R (9), t (3), 1/fx, 1/fy, cx, cy, mean focal
+// a / b, rounded as the division rounds it, from b's reciprocal r to within an ulp: the product's error goes
+// through r once more (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990). Short of overflow and underflow, which a camera's and a scene's sizes stay far from.
+__device__ inline double quotient(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-q, b, a), r, q);
+}
+// b's reciprocal to within an ulp: the instruction's estimate and two Newton steps.
+__device__ inline double reciprocal(double b) {
+  double r = __builtin_amdgcn_rcp(b);
+  for (int k = 0; k < 2; ++k) r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+  return r;
+}
+constexpr int CAMS = 64, CAMLD = 19;  // R (9), t (3), 1/fx, 1/fy, cx, cy, mean focal, fx, fy
 template <bool LDSCAM, typename I, bool LAZY>
 __global__ void __launch_bounds__(256) recon_points_kernel(
     int V, int H, int W, int bpv, const float* __restrict__ depth, const float* __restrict__ pts_cam,
@@ -1337,6 +1351,8 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
     for (int k = 0; k < 12; ++k) d[k] = c[k];
     for (int k = 14; k < 16; ++k) d[k] = c[k];
     d[16] = (c[12] + c[13]) / 2.0;  // before 12 and 13: c may be d
+    d[17] = c[12];
+    d[18] = c[13];
     d[12] = 1.0 / c[12];
     d[13] = 1.0 / c[13];
   };
@@ -1373,8 +1389,8 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
     double p[3];
     if (depth) {
       const double d = depth[id];
-      p[0] = (x - own[14]) * own[12] * d;
-      p[1] = (y - own[15]) * own[13] * d;
+      p[0] = quotient(x - own[14], own[17], own[12]) * d;
+      p[1] = quotient(y - own[15], own[18], own[13]) * d;
       p[2] = d;
     } else {
       for (int k = 0; k < 3; ++k) p[k] = pts_cam[id * 3 + k];
@@ -1400,8 +1416,8 @@ __global__ void __launch_bounds__(256) recon_points_kernel(
         if (!(qz > 0.0)) continue;
         const double qx = c[0] * dx + c[3] * dy + c[6] * dz;
         const double qy = c[1] * dx + c[4] * dy + c[7] * dz;
-        const double r = 1.0 / qz;
-        const double u = c[16] * qx * r + c[14], w = c[16] * qy * r + c[15];
+        const double r = reciprocal(qz);
+        const double u = quotient(c[16] * qx, qz, r) + c[14], w = quotient(c[16] * qy, qz, r) + c[15];
         // round(u) in [0, W): u in (-0.5, W - 0.5), and there half away from zero is half up
         if (!(u > -0.5 && w > -0.5 && u < fW && w < fH)) continue;
         const double uf = floor(u), wf = floor(w);

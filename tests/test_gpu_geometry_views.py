@@ -74,6 +74,41 @@ def test_points_over_their_source(ctx):
     assert 0 < int((ref[2] == 0).sum()) < conf.numel()
 
 
+def test_half_pixels_round_away_from_zero(ctx):
+    """Every projection of view 0 into view 1 lies exactly half way between two columns (focal length 64, depths
+    that divide 43065, a translation of 43065 / 128: all exact in fp32, and the fitted intrinsics in f64),
+    and view 1's columns are in turn more and less confident: the confidences are f64::round's."""
+    Z = 43065
+    z = np.array([d for d in range(1, Z + 1, 2) if Z % d == 0 and Z // d < 90], np.float64)
+    H, W, cx = len(z), 48, 24.0
+    cy = H / 2
+    rows, cols = np.meshgrid(np.arange(H), np.arange(W), indexing="ij")
+    pts = np.empty((2, H, W, 3), np.float32)
+    for v, k in ((0, 1), (1, 4)):   # view 1 sees everything four times as far
+        depth = k * z[:, None] * np.ones((1, W))
+        pts[v] = np.stack([(cols - cx) * depth / 64, (rows - cy) * depth / 64, depth], -1)
+    conf = np.full((2, H, W), 2.0, np.float32)
+    conf[1] = np.where(cols % 2, 3.0, 1.0)
+    trans = np.zeros((2, 3), np.float32)
+    trans[1, 0] = Z / 128
+    quat = np.tile(np.array([0, 0, 0, 1], np.float32), (2, 1))
+    d = {k: torch.from_numpy(a).cuda() for k, a in (("points_in_camera", pts), ("quaternion", quat), ("translation", trans),
+                                                    ("conf", conf), ("mask", np.ones((2, H, W), np.uint8)))}
+    cams = torch.empty(2, 16, dtype=torch.float64, device="cuda")
+    points, out = torch.empty(2, H, W, 3, device="cuda"), torch.empty(2, H, W, device="cuda")
+    torch.cuda.synchronize()
+    ctx.kernel_reconstruct(2, H, W, **{k: t.data_ptr() for k, t in d.items()}, cameras=cams.data_ptr(),
+                           points=points.data_ptr(), conf_out=out.data_ptr())
+    ctx.synchronize()
+    assert cams[:, 12:].tolist() == [[64.0, 64.0, cx, cy]] * 2
+    twice = 2 * cols - (Z / z).astype(int)[:, None]            # 2 u, odd
+    column = np.where(twice >= 0, (twice + 1) // 2, (twice - 1) // 2)
+    seen = (column >= 0) & (column < W)
+    want = conf.copy()
+    want[0][seen & (column % 2 == 1)] = 0.0
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("H,W", [(46340, 46340), (46342, 46341)])   # within a turn of 2^31 pixels, and past it
 def test_largest_view(ctx, H, W):
     """One view whose pixel numbers pass 32 bits on the last turn, or are longer: every confidence is kept, and
