@@ -99,7 +99,8 @@ int splat_kernel_resize_bilinear(splat_ctx* ctx, int dtype, const void* in, int 
  * pose_encoding [V,9]); MapAnything mode otherwise (points_in_camera [V,H,W,3], quaternion
  * [V,4] xyzw, translation [V,3], mask [V,H,W] u8 unambiguous). conf [V,H,W]; foreground
  * [V,H,W] u8 or NULL. Out: cameras [V,16] f64 (R row-major, t, fx, fy, cx, cy, view 0's
- * frame), points [V,H,W,3], conf_out [V,H,W]. */
+ * frame), points [V,H,W,3], conf_out [V,H,W]. An input may share memory with an output (conf
+ * cleaned in place, say): it is read from a copy that the context keeps. */
 int splat_kernel_reconstruct(splat_ctx* ctx, int V, int H, int W, const float* depth, const float* pose_encoding,
                              const float* points_in_camera, const float* quaternion, const float* translation,
                              const float* conf, const uint8_t* mask, const uint8_t* foreground, double* cameras,

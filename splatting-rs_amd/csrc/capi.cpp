@@ -4,6 +4,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
+#include <type_traits>
 
 #include "runtime.h"
 #include "../../include/splathip_kernels.h"
@@ -566,18 +568,37 @@ int splat_kernel_reconstruct(splat_ctx* ctx, int V, int H, int W, const float* d
   return guard(c, [&] {
     SPLAT_CHECK(V > 0 && H > 0 && W > 0 && conf && cameras && points && conf_out, BAD_ARGUMENT, "geometry args");
     const size_t px = size_t(V) * H * W;
-    // the cleaning compares the given confidences of other pixels: in place, it reads a copy
-    if (conf < conf_out + px && conf_out < conf + px) {
-      float* copy = static_cast<float*>(staging(c, 21, px * 4));
-      convert(c->ex, F32, conf, F32, copy, long(px));
-      conf = copy;
+    // Every block reads inputs of other pixels while others store: an input that shares memory with an
+    // output is read from a copy (confidences cleaned in place, points over the points they come from).
+    struct Range { const char* at; size_t bytes; };
+    const Range outs[] = {{reinterpret_cast<const char*>(cameras), size_t(V) * 16 * 8},
+                          {reinterpret_cast<const char*>(points), px * 12},
+                          {reinterpret_cast<const char*>(conf_out), px * 4}};
+    int slot = 60;  // staging slots of their own
+    auto apart = [&](auto& in, size_t count) {
+      using T = std::remove_cv_t<std::remove_pointer_t<std::remove_reference_t<decltype(in)>>>;
+      ++slot;
+      const char* q = reinterpret_cast<const char*>(in);
+      const size_t bytes = count * sizeof(T);
+      if (!q || std::none_of(std::begin(outs), std::end(outs),
+                             [&](const Range& o) { return q < o.at + o.bytes && o.at < q + bytes; }))
+        return;
+      void* copy = staging(c, slot, bytes);
+      if constexpr (sizeof(T) == 4) convert(c->ex, F32, in, F32, copy, long(count));
+      else SPLAT_HIP(hipMemcpyAsync(copy, in, bytes, hipMemcpyDeviceToDevice, c->stream));
+      in = static_cast<const T*>(copy);
+    };
+    apart(conf, px);
+    apart(foreground, px);
+    if (depth) {
+      apart(depth, px);
+      apart(pose_encoding, size_t(V) * 9);
+    } else {
+      apart(points_in_camera, px * 3);
+      apart(quaternion, size_t(V) * 4);
+      apart(translation, size_t(V) * 3);
     }
-    // and other pixels' depths: points over the points they come from
-    if (points_in_camera && points_in_camera < points + 3 * px && points < points_in_camera + 3 * px) {
-      float* copy = static_cast<float*>(staging(c, 22, px * 12));
-      convert(c->ex, F32, points_in_camera, F32, copy, long(px) * 3);
-      points_in_camera = copy;
-    }
+    apart(mask, px);
     double* d_fit = depth ? nullptr : static_cast<double*>(staging(c, 24, size_t(V) * 4 * 8));
     reconstruct_geometry(c->ex, V, H, W, depth, pose_encoding, points_in_camera, quaternion, translation, conf, mask,
                          foreground, cameras, d_fit, points, conf_out);

@@ -74,6 +74,49 @@ def test_points_over_their_source(ctx):
     assert 0 < int((ref[2] == 0).sum()) < conf.numel()
 
 
+@pytest.mark.parametrize("mode,inputs,over", [
+    ("da3", ("pose_encoding",), "points"), ("da3", ("foreground", "pose_encoding"), "conf_out"), ("da3", ("depth",), "points"),
+    ("da3", ("conf",), "points"), ("ma", ("mask", "foreground"), "conf_out"), ("ma", ("quaternion", "translation"), "points"),
+    ("ma", ("mask", "quaternion"), "points"), ("ma", ("translation",), "cameras"),
+])
+def test_inputs_in_an_output_s_memory(ctx, mode, inputs, over):
+    """Inputs that lie, one after the other and off its start, in an output's memory: what separate buffers give."""
+    V, H, W = 3, 70, 98
+    g = torch.Generator().manual_seed(3)
+    z = 2 + 0.2 * torch.randn(V, H, W, generator=g)
+    conf = 1 + torch.exp(torch.randn(V, H, W, generator=g))
+    fg = (torch.rand(V, H, W, generator=g) < 0.9).to(torch.uint8)
+    shift = torch.randn(V, 3, generator=g).mul(0.05)
+    turn = torch.cat([torch.randn(V, 3, generator=g).mul(0.02), torch.ones(V, 1)], 1)
+    if mode == "da3":
+        d = {"depth": z, "pose_encoding": torch.cat([shift, turn, torch.full((V, 2), 0.9)], 1), "conf": conf, "foreground": fg}
+    else:
+        y, x = torch.meshgrid(torch.linspace(-0.4, 0.4, H), torch.linspace(-0.5, 0.5, W), indexing="ij")
+        d = {"points_in_camera": torch.stack([x * z, y * z, z], -1), "quaternion": turn, "translation": shift, "conf": conf,
+             "mask": (torch.rand(V, H, W, generator=g) < 0.9).to(torch.uint8), "foreground": fg}
+    d = {k: t.contiguous().cuda() for k, t in d.items()}
+
+    def call(shared):
+        out = {"cameras": torch.zeros(V, 16, dtype=torch.float64, device="cuda"), "points": torch.zeros(V, H, W, 3, device="cuda"),
+               "conf_out": torch.zeros(V, H, W, device="cuda")}
+        ptr = {k: t.data_ptr() for k, t in {**d, **out}.items()}
+        at = 16
+        for k in inputs if shared else ():
+            raw = out[over].view(-1).view(torch.uint8)
+            n = d[k].numel() * d[k].element_size()
+            raw[at:at + n] = d[k].reshape(-1).view(torch.uint8)
+            ptr[k] = raw.data_ptr() + at
+            at += (n + 15) // 16 * 16
+        torch.cuda.synchronize()
+        ctx.kernel_reconstruct(V, H, W, **ptr)
+        ctx.synchronize()
+        return out
+
+    want, got = call(False), call(True)
+    assert 0 < int((want["conf_out"] == 0).sum()) < conf.numel()
+    assert all(torch.equal(want[k], got[k]) for k in want)
+
+
 def test_half_pixels_round_away_from_zero(ctx):
     """Every projection of view 0 into view 1 lies exactly half way between two columns (focal length 64, depths
     that divide 43065, a translation of 43065 / 128: all exact in fp32, and the fitted intrinsics in f64),
