@@ -6,14 +6,14 @@
 // (mapanything-rs/src/image_input.rs:195-216).
 #include <algorithm>
 #include <array>
-#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
-#include <system_error>
+#include <sched.h>
 #include <thread>
 #include <vector>
 
+#include "ring_fill.h"
 #include "runtime.h"
 
 namespace splat {
@@ -74,56 +74,17 @@ struct Photo {
   int left, top;
 };
 
-// Worker threads that copy a list of host images, cut into chunks, into the pinned ring in order;
-// the calling thread hands each finished chunk to the GPU and frees ring slots as their copies end.
-class RingFill {
- public:
-  struct Chunk { const uint8_t* src; size_t bytes; };
-  RingFill(uint8_t* ring, std::vector<Chunk> chunks) : ring_(ring), chunks_(std::move(chunks)), done_(chunks_.size()) {
-    for (auto& d : done_) d.store(false, std::memory_order_relaxed);
-    allowed_.store(HostRing::SLOTS);
-    try {
-      for (int t = 0; t < HostRing::THREADS; ++t) threads_.emplace_back([this] { work(); });
-    } catch (const std::system_error&) {  // fewer threads than asked for: see take()
-    }
-  }
-  ~RingFill() {
-    stop_.store(true);
-    for (auto& t : threads_) t.join();
-  }
-  bool filled(size_t i) const { return done_[i].load(std::memory_order_acquire); }
-  void free_one() { allowed_.fetch_add(1, std::memory_order_release); }
-  // With no worker at all the calling thread copies.
-  void help() { if (threads_.empty()) take(); }
-
- private:
-  bool take() {
-    size_t i = next_.load();
-    do {
-      if (i >= chunks_.size() || i >= allowed_.load(std::memory_order_acquire)) return false;
-    } while (!next_.compare_exchange_weak(i, i + 1));
-    std::memcpy(ring_ + (i % HostRing::SLOTS) * HostRing::CHUNK, chunks_[i].src, chunks_[i].bytes);
-    done_[i].store(true, std::memory_order_release);
-    return true;
-  }
-  void work() {
-    while (!stop_.load() && next_.load() < chunks_.size())
-      if (!take()) std::this_thread::yield();
-  }
-  uint8_t* ring_;
-  std::vector<Chunk> chunks_;
-  std::vector<std::atomic<bool>> done_;
-  std::atomic<size_t> next_{0}, allowed_{0};
-  std::atomic<bool> stop_{false};
-  std::vector<std::thread> threads_;
-};
+// CPUs that this process may run on.
+int usable_cpus() {
+  cpu_set_t set;
+  return sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : int(std::thread::hardware_concurrency());
+}
 
 // Resizes and crops every photo into `batch` [n, ch, cw, 4]. The resize weights of all of them are
-// computed once per (size, filter) and uploaded together; the pixels go up through the pinned ring
-// on the second stream into one of two device buffers while the previous photo is resized.
-// The host pixels have been read on return; the caller synchronises c.stream. Six 12 MB photos: 4.0 -> 2.1 ms
-// (uploads of pageable memory one after the other at 26 GB/s, weights computed for every photo, a
-// synchronisation after each step).
+// computed once per (size, filter) and uploaded together; the pixels go up on the second stream into one of
+// two device buffers while the previous photo is resized, through the pinned ring. The caller synchronises c.stream, and the host pixels have been read then.
+// Six 12 MB photos: 4.0 -> 2.1 ms (uploads of pageable memory one after the other at 26 GB/s, weights
+// computed for every photo, a synchronisation after each step).
 void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, uint8_t* batch) {
   size_t src_bytes = 0, out_bytes = 0, tmp_bytes = 0, total = 0;
   for (const Photo& p : photos) {
@@ -204,8 +165,9 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
     }
     crop_into(c, cur, w, p.left, p.top, cw, ch, batch + k * size_t(cw) * ch * 4);
   };
-  // A few small photos: the ring's threads cost more than they save.
-  if (total < (size_t(2) << 20)) {
+  // A few small photos, where the ring's threads cost more than they save; or a single CPU, whose one
+  // thread the driver's own staging serves as well (one 12 MB photo 580 us, through the ring 670).
+  if (total < (size_t(2) << 20) || usable_cpus() < 2) {
     make_taps();
     for (size_t k = 0; k < photos.size(); ++k) {
       SPLAT_HIP(hipMemcpyAsync(src[k & 1], photos[k].host, size_t(photos[k].w) * photos[k].h * 4, hipMemcpyHostToDevice, c.stream));
@@ -215,15 +177,15 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
   }
   HostRing& ring = c.host_ring();
   std::vector<RingFill::Chunk> chunks;
-  for (const Photo& p : photos) {
-    const size_t bytes = size_t(p.w) * p.h * 4;
-    for (size_t o = 0; o < bytes; o += HostRing::CHUNK)
-      chunks.push_back({p.host + o, std::min(HostRing::CHUNK, bytes - o)});
+  for (size_t k = 0; k < photos.size(); ++k) {
+    const size_t bytes = size_t(photos[k].w) * photos[k].h * 4;
+    for (size_t o = 0; o < bytes; o += RingFill::CHUNK)
+      chunks.push_back({photos[k].host + o, std::min(RingFill::CHUNK, bytes - o)});
   }
   // the copies start after what c.stream holds (an earlier call's readers of `src`)
   SPLAT_HIP(hipEventRecord(ring.used[0], c.stream));
   SPLAT_HIP(hipStreamWaitEvent(c.aux, ring.used[0], 0));
-  RingFill fill(ring.base, chunks);
+  RingFill fill(ring.base, std::move(chunks));
   struct Drain {  // the ring is free again on return, also when an error leaves early
     Context& c;
     ~Drain() { (void)hipStreamSynchronize(c.aux); }
@@ -232,21 +194,27 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
   auto hand_over = [&](size_t k) {
     if (k >= 2) SPLAT_HIP(hipStreamWaitEvent(c.aux, ring.used[k & 1], 0));  // photo k - 2 has been read
     const size_t bytes = size_t(photos[k].w) * photos[k].h * 4;
-    for (size_t at = 0; at < bytes; at += chunks[i++].bytes) {
+    for (size_t at = 0; at < bytes; at += fill.bytes(i++)) {
       while (!fill.filled(i)) {
-        fill.help();
-        const hipError_t e = landed < i ? hipEventQuery(ring.sent[landed % HostRing::SLOTS]) : hipErrorNotReady;
-        if (e == hipErrorNotReady) {
-          (void)hipGetLastError();  // no error: the launches below ask for theirs
-          std::this_thread::yield();
-        } else {
-          SPLAT_HIP(e);
-          ++landed;
-          fill.free_one();
+        if (fill.help()) continue;
+        if (landed < i) {
+          hipError_t e = hipEventQuery(ring.sent[landed % RingFill::SLOTS]);
+          if (e == hipErrorNotReady) {
+            (void)hipGetLastError();  // no error: the launches below ask for theirs
+            // the ring is full: nothing moves before this copy has ended
+            if (!fill.has_room(i)) e = hipEventSynchronize(ring.sent[landed % RingFill::SLOTS]);
+          }
+          if (e != hipErrorNotReady) {
+            SPLAT_HIP(e);
+            ++landed;
+            fill.free_one();
+            continue;
+          }
         }
+        std::this_thread::yield();  // a worker is copying the chunk, 2 MB
       }
-      const size_t slot = i % HostRing::SLOTS;
-      SPLAT_HIP(hipMemcpyAsync(src[k & 1] + at, ring.base + slot * HostRing::CHUNK, chunks[i].bytes, hipMemcpyHostToDevice, c.aux));
+      const size_t slot = i % RingFill::SLOTS;
+      SPLAT_HIP(hipMemcpyAsync(src[k & 1] + at, ring.base + slot * RingFill::CHUNK, fill.bytes(i), hipMemcpyHostToDevice, c.aux));
       SPLAT_HIP(hipEventRecord(ring.sent[slot], c.aux));
     }
     SPLAT_HIP(hipEventRecord(ring.copied[k & 1], c.aux));

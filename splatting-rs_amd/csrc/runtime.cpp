@@ -584,7 +584,7 @@ void* Context::staging_buffer(int slot, size_t bytes) {
 
 HostRing::HostRing() {
   try {
-    SPLAT_HIP(hipHostMalloc(reinterpret_cast<void**>(&base), SLOTS * CHUNK, hipHostMallocDefault));
+    SPLAT_HIP(hipHostMalloc(reinterpret_cast<void**>(&base), RingFill::SLOTS * RingFill::CHUNK, hipHostMallocDefault));
     for (hipEvent_t& e : sent) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (hipEvent_t& e : copied) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (hipEvent_t& e : used) SPLAT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -596,7 +596,7 @@ HostRing::HostRing() {
 
 HostRing::~HostRing() {
   for (hipEvent_t* e : {&sent[0], &copied[0], &used[0]}) {
-    const int n = e == &sent[0] ? SLOTS : 2;
+    const int n = e == &sent[0] ? RingFill::SLOTS : 2;
     for (int k = 0; k < n; ++k)
       if (e[k]) (void)hipEventDestroy(e[k]);
   }

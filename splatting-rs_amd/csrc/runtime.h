@@ -11,6 +11,7 @@
 #include "../../include/splathip.h"
 #include "host_tables.h"
 #include "kernels.h"
+#include "ring_fill.h"
 #include "safetensors.h"
 
 namespace splat {
@@ -293,14 +294,11 @@ class MaModel {
 
 // --- context ---------------------------------------------------------------------------------
 
-// Pinned host memory that pageable photos go to the GPU through, in chunks, several threads filling
-// it (one thread copies at about half the link's rate): SLOTS chunks in flight. `sent`: a slot's
+// Pinned host memory that pageable photos go to the GPU through, RingFill's chunks. `sent`: a slot's
 // copy; `copied` / `used`: a photo's device buffer written / read (two of them in turn).
 struct HostRing {
-  static constexpr size_t CHUNK = size_t(2) << 20;
-  static constexpr int SLOTS = 8, THREADS = 3;
   uint8_t* base = nullptr;
-  hipEvent_t sent[SLOTS] = {}, copied[2] = {}, used[2] = {};
+  hipEvent_t sent[RingFill::SLOTS] = {}, copied[2] = {}, used[2] = {};
   HostRing();
   ~HostRing();
 };

@@ -1,7 +1,9 @@
 """Photo batches through the pinned upload ring (16 MB in 2 MB chunks, two device buffers in turn):
-batches that wrap it, end in part of a chunk, hold one photo or photos of several sizes, and one
-below the ring's threshold. Each photo must come out as the single-image resize (itself checked
-against the oracle in tests/test_gpu_preprocess.py) gives it, byte for byte."""
+batches that wrap it, end in part of a chunk, hold one photo or photos of several sizes, and one below the ring's threshold; MapAnything's inputs (one resize a photo) and DA3's
+(two, which alternate between two buffers). Each photo must come out as the single-image resizes (themselves
+checked against the oracle in tests/test_gpu_preprocess.py) give it, byte for byte."""
+import os
+
 import numpy as np
 import pytest
 
@@ -42,3 +44,68 @@ def test_batches(ctx, sizes):
             want, want_fg = to_model_input(np.ascontiguousarray(r[None, top:top + H, left:left + W]))
             assert np.array_equal(img[k].cpu().numpy(), want[0]), k
             assert np.array_equal(fg[k].cpu().numpy().astype(bool), want_fg[0]), k
+
+
+DA3_SIZES = [(2100, 1403), (1201, 1900), (2000, 1300), (1600, 1100)]   # 38 MB, every size of its own
+
+
+def _photos(sizes, pinned=()):
+    rng = np.random.default_rng(len(sizes))
+    photos = []
+    for k, (w, h) in enumerate(sizes):
+        p = torch.empty(h, w, 4, dtype=torch.uint8, pin_memory=k in pinned).numpy()
+        p[:] = rng.integers(0, 256, size=(h, w, 4), dtype=np.uint8)
+        p[..., 3] |= 128
+        photos.append(p)
+    return photos
+
+
+def _da3(ctx, photos):
+    W, H = splathip.da3_model_inputs_size([(p.shape[1], p.shape[0]) for p in photos])
+    img = torch.zeros(len(photos), 3, H, W, device="cuda")
+    fg = torch.zeros(len(photos), H, W, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert ctx.da3_model_inputs_device(photos, img.data_ptr(), fg.data_ptr()) == (H, W)
+    ctx.synchronize()
+    return img.cpu().numpy(), fg.cpu().numpy()
+
+
+def _da3_one_by_one(ctx, photos):
+    """The two resizes of each photo through splat_resize_rgba8, then the common crop."""
+    W, H = splathip.da3_model_inputs_size([(p.shape[1], p.shape[0]) for p in photos])
+    out = []
+    for p in photos:
+        (bw, bh), (w, h) = P.model_input_size(p.shape[1], p.shape[0])
+        resized = 0
+        for nw, nh in ((bw, bh), (w, h)):
+            if (p.shape[1], p.shape[0]) != (nw, nh):
+                f = P.CATMULLROM if nw > p.shape[1] or nh > p.shape[0] else P.TRIANGLE
+                p = ctx.resize_rgba8(np.ascontiguousarray(p), nw, nh, f)
+                resized += 1
+        assert resized == 2
+        left, top = (w - W) // 2, (h - H) // 2
+        out.append(to_model_input(np.ascontiguousarray(p[None, top:top + H, left:left + W])))
+    return out
+
+
+def test_da3_batches(ctx):
+    photos = _photos(DA3_SIZES)
+    want = _da3_one_by_one(ctx, photos)
+    for _ in range(2):
+        img, fg = _da3(ctx, photos)
+        for k in range(len(photos)):
+            assert np.array_equal(img[k], want[k][0][0]), k
+            assert np.array_equal(fg[k].astype(bool), want[k][1][0]), k
+
+
+def test_one_cpu(ctx):
+    """With a single CPU to run on, pageable photos go without the ring: the same bytes."""
+    photos = _photos(DA3_SIZES)
+    want = _da3(ctx, photos)
+    cpus = os.sched_getaffinity(0)
+    os.sched_setaffinity(0, {min(cpus)})
+    try:
+        got = _da3(ctx, photos)
+    finally:
+        os.sched_setaffinity(0, cpus)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])

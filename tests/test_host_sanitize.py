@@ -126,3 +126,27 @@ def test_host_tables_and_size_rules(harness):
     assert res["da3_size 4032x3024"].endswith("OK 504 378 504 378")
     assert res["ma_size 1000x700"].endswith("OK 518x392 cover 560x392")
     assert res["pos 1 37x37"].split(" OK ")[1].startswith("1370 ")
+
+
+@pytest.fixture(scope="module")
+def ring(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ is not installed")
+    out = str(tmp_path_factory.mktemp("ring") / "ring_fill_main")
+    cmd = [gxx, "-std=c++17", "-O1", "-g", "-pthread", "-fsanitize=thread", os.path.join(ROOT, "tests", "host", "ring_fill_main.cpp"),
+           "-o", out]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
+    return out
+
+
+@pytest.mark.parametrize("mode,sizes,said", [
+    ("whole", "0", "ok"), ("whole", "1", "ok"), ("whole", "2097152", "ok"), ("whole", "2097153,5,4194304", "ok"),
+    ("whole", "12582912,12582912,12582912", "ok"),            # wraps the eight slots
+    ("abandon", "12582912,12582912", "abandoned"),            # an error leaves early, workers still copying
+])
+def test_photo_ring_under_thread_sanitizer(ring, mode, sizes, said):
+    for _ in range(3):
+        r = subprocess.run([ring, mode, sizes], capture_output=True, text=True, timeout=60)
+        assert "ThreadSanitizer" not in r.stderr, r.stderr[-3000:]
+        assert r.returncode == 0 and r.stdout.split() == [said]
