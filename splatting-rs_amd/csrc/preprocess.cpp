@@ -80,9 +80,20 @@ int usable_cpus() {
   return sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : int(std::thread::hardware_concurrency());
 }
 
+// Memory that the GPU cannot read by itself (not page-locked, managed or device memory).
+bool pageable(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
 // Resizes and crops every photo into `batch` [n, ch, cw, 4]. The resize weights of all of them are
 // computed once per (size, filter) and uploaded together; the pixels go up on the second stream into one of
-// two device buffers while the previous photo is resized, through the pinned ring. The caller synchronises c.stream, and the host pixels have been read then.
+// two device buffers while the previous photo is resized, pageable ones through the pinned ring,
+// page-locked ones as they lie. The caller synchronises c.stream, and the host pixels have been read then.
 // Six 12 MB photos: 4.0 -> 2.1 ms (uploads of pageable memory one after the other at 26 GB/s, weights
 // computed for every photo, a synchronisation after each step).
 void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, uint8_t* batch) {
@@ -165,9 +176,15 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
     }
     crop_into(c, cur, w, p.left, p.top, cw, ch, batch + k * size_t(cw) * ch * 4);
   };
+  std::vector<bool> direct;
+  size_t staged = 0;  // bytes for the ring
+  for (const Photo& p : photos) {
+    direct.push_back(!pageable(p.host));
+    if (!direct.back()) staged += size_t(p.w) * p.h * 4;
+  }
   // A few small photos, where the ring's threads cost more than they save; or a single CPU, whose one
   // thread the driver's own staging serves as well (one 12 MB photo 580 us, through the ring 670).
-  if (total < (size_t(2) << 20) || usable_cpus() < 2) {
+  if (total < (size_t(2) << 20) || (staged > 0 && usable_cpus() < 2)) {
     make_taps();
     for (size_t k = 0; k < photos.size(); ++k) {
       SPLAT_HIP(hipMemcpyAsync(src[k & 1], photos[k].host, size_t(photos[k].w) * photos[k].h * 4, hipMemcpyHostToDevice, c.stream));
@@ -179,7 +196,7 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
   std::vector<RingFill::Chunk> chunks;
   for (size_t k = 0; k < photos.size(); ++k) {
     const size_t bytes = size_t(photos[k].w) * photos[k].h * 4;
-    for (size_t o = 0; o < bytes; o += RingFill::CHUNK)
+    for (size_t o = 0; !direct[k] && o < bytes; o += RingFill::CHUNK)
       chunks.push_back({photos[k].host + o, std::min(RingFill::CHUNK, bytes - o)});
   }
   // the copies start after what c.stream holds (an earlier call's readers of `src`)
@@ -194,7 +211,8 @@ void resize_batch(Context& c, const std::vector<Photo>& photos, int cw, int ch, 
   auto hand_over = [&](size_t k) {
     if (k >= 2) SPLAT_HIP(hipStreamWaitEvent(c.aux, ring.used[k & 1], 0));  // photo k - 2 has been read
     const size_t bytes = size_t(photos[k].w) * photos[k].h * 4;
-    for (size_t at = 0; at < bytes; at += fill.bytes(i++)) {
+    if (direct[k]) SPLAT_HIP(hipMemcpyAsync(src[k & 1], photos[k].host, bytes, hipMemcpyHostToDevice, c.aux));
+    for (size_t at = 0; !direct[k] && at < bytes; at += fill.bytes(i++)) {
       while (!fill.filled(i)) {
         if (fill.help()) continue;
         if (landed < i) {

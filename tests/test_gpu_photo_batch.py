@@ -1,5 +1,6 @@
 """Photo batches through the pinned upload ring (16 MB in 2 MB chunks, two device buffers in turn):
-batches that wrap it, end in part of a chunk, hold one photo or photos of several sizes, and one below the ring's threshold; MapAnything's inputs (one resize a photo) and DA3's
+batches that wrap it, end in part of a chunk, hold one photo or photos of several sizes, page-locked ones
+among them, and one below the ring's threshold; MapAnything's inputs (one resize a photo) and DA3's
 (two, which alternate between two buffers). Each photo must come out as the single-image resizes (themselves
 checked against the oracle in tests/test_gpu_preprocess.py) give it, byte for byte."""
 import os
@@ -88,14 +89,30 @@ def _da3_one_by_one(ctx, photos):
     return out
 
 
-def test_da3_batches(ctx):
-    photos = _photos(DA3_SIZES)
+@pytest.mark.parametrize("pinned", [(), (0, 1, 2, 3), (1,), (0, 2)])
+def test_da3_batches(ctx, pinned):
+    photos = _photos(DA3_SIZES, pinned)
     want = _da3_one_by_one(ctx, photos)
     for _ in range(2):
         img, fg = _da3(ctx, photos)
         for k in range(len(photos)):
             assert np.array_equal(img[k], want[k][0][0]), k
             assert np.array_equal(fg[k].astype(bool), want[k][1][0]), k
+
+
+def test_host_pixels_are_read_on_return(ctx):
+    """Page-locked photos, below and above the ring's threshold, overwritten as soon as the call returns."""
+    for sizes in (DA3_SIZES[:2], [(300, 260), (280, 300)]):
+        photos = _photos(sizes, range(len(sizes)))
+        want = _da3(ctx, photos)
+        W, H = splathip.da3_model_inputs_size([(p.shape[1], p.shape[0]) for p in photos])
+        img = torch.zeros(len(photos), 3, H, W, device="cuda")
+        torch.cuda.synchronize()
+        ctx.da3_model_inputs_device(photos, img.data_ptr())
+        for p in photos:
+            p[:] = 255
+        ctx.synchronize()
+        assert np.array_equal(img.cpu().numpy(), want[0])
 
 
 def test_one_cpu(ctx):
