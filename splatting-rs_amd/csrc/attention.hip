@@ -1134,20 +1134,25 @@ static int attn_splits(long blocks, int ntiles, bool qt2) {
 }
 
 // Key slices of an fp32 launch of `blocks` blocks of 128 queries, `ntiles` 32-key tiles each; S <= 8,
-// at least 2 tiles a slice. A CU with n slices takes n x 0.7 of one slice's time (1 for n = 1: two
-// blocks share a CU), a slice its tiles plus about 3 tiles' worth of start, partials and merge.
-// Taken when 5% below the unsplit launch. The partials stay within ATTN_SCRATCH_BYTES, so that the
-// allocation-free entry point takes the same plan. Measured, us for S = 1 .. 8: 1297 tokens x 6
-// heads 71 44 35 37 36 34 32 33; 6 x 973 x 6 82 79 75 78 81 82 85 88; 5838 x 6 412 378 322 319 305
-// 304 303 300; 2593 x 12 139 122 130 127 132 132 135 141; 8 x 1297 x 16 321 330 353 373 391 ...
+// at least 2 tiles a slice: the cheapest by a model of the time in us, 3.8 and 1.65 a tile of one
+// block on its CU (two blocks share a CU: 1.35 to 1.6 times that, more 0.5 + 0.8 times their number a
+// CU); slices add a merge, 4 us and 0.4 a MB of partials, 0.15 past 15 MB. The partials stay within
+// ATTN_SCRATCH_BYTES, so that the allocation-free entry point takes the same plan. Measured, us for S = 1
+// .. 8: 1297 tokens x 6 heads 70 43 34 34 33 31 30 29; 6 x 973 x 6 76 77 68 71 74 74 79 80; 5838 x 6 415 376
+// 319 313 301 300 300 295; 2593 x 12 140 120 127 125 130 129 133 138; 8 x 181 x 16 15 22 26; 8 x 97 x 16
+// 11.4 14.3; 1 x 325 x 6 22.7 17.4 14.5 13.3. 23 such shapes: 28.8 us by the rule, 28.6 at best.
 static int attn_f32_splits(long blocks, int ntiles, long rows) {
   int best = 1;
   double bc = 1e30;
   for (int S = 1; S <= ATTN_MAX_SPLITS; ++S) {
+    const double mb = double(S) * double(rows) * (64 + 2) * sizeof(float) * 1e-6;
     if (S > 1 && (ntiles / S < 2 || size_t(S) * rows * (64 + 2) * sizeof(float) > ATTN_SCRATCH_BYTES)) break;
-    const long n = (blocks * S + 255) / 256;
-    const double cost = (n == 1 ? 1.0 : 0.7 * double(n)) * (double(ntiles) / S + 3.0) * (S > 1 ? 1.05 : 1.0);
-    if (cost < bc * 0.999) { bc = cost; best = S; }
+    const int tps = cdiv(ntiles, S);
+    const double x = double(blocks) * cdiv(ntiles, tps) / 256.0;  // blocks a CU
+    const double share = x <= 1.0 ? 1.0 : x <= 2.0 ? 1.35 + 0.27 * (x - 1.0) : 0.5 + 0.8 * x;
+    double t = 3.8 + 1.65 * tps * share;
+    if (S > 1) t = 1.03 * (t + 4.0 + 0.4 * std::min(mb, 15.0) + 0.15 * std::max(mb - 15.0, 0.0));
+    if (t < bc * 0.999) { bc = t; best = S; }
   }
   return best;
 }

@@ -1654,13 +1654,13 @@ static size_t split_bytes(const GemmArgs& a, int S) {
 // matrix cores, 32x32 (64x64 tiles) by the VALU. The plan, a tile and a number of K slices (not for
 // 128x64), is the cheapest by a model of the time in us: start + tile * n + (32-element k-tiles of a
 // slice) * step, n the blocks of the fullest CU, step with one block a CU (the chip full: more, in
-// proportion to its fill), n steps of `steps` with several; slices add a reduce, 4.3 us and 0.16 a MB
-// of partials. Constants fitted to 103 shapes, every tile, 1 to 16 slices: the choices' geometric mean is
-// 25.0 us, the measured best's 24.8.
+// proportion to its fill), n steps of `steps` with several; slices add a reduce, 3.2 us, 0.3 a slice
+// (their loads follow one another) and 0.16 a MB of partials. Constants fitted to 167 shapes, every tile, 1
+// to 16 slices: the choices' geometric mean is 17.8 us, the measured best's 17.8.
 // Measured, us (64x64 / 128x64 / 128x128, "in S" with the reduce): 1297x384x384 9.6 (11.9 in 2) / 13.9 /
 // 17.5; 1297x384x1536 28.3 (21.3 in 2, 21.8 in 4) / 43.8 / 55.7; 1297x1152x384 14.6 / 15.4 / 18.4;
 // 3892x384x1536 45.6 (43.4 in 2) / 46.7 / 56.7 (40.4 in 2); 5838x1152x384 45.5 / 44.3 / 35.0; 5838x384x1536
-// 67.5 / 74.2 / 58.3 (52.1 in 3); 3x3 of 64 channels, 23328 pixels 22.7 / 24.9, 5184 pixels 16.1 (13.9 in
+// 67.5 / 74.2 / 58.3 (52.1 in 3); 65x384x2048 35.7 (12.7 in 8, 13.5 in 16); 3x3 of 64 channels, 23328 pixels 22.7 / 24.9, 5184 pixels 16.1 (13.9 in
 // 3); 2x2 transposed convolution of 96 channels on 6 x 27x36 10.9 / 12.8 / 15.0.
 struct F32Plan { BfCfg cfg; int S; };
 struct F32Cost {
@@ -1695,7 +1695,7 @@ struct F32Cost {
       double t = (f ? c.start_full : conv ? c.start_conv : c.start) + double(n) * (!f ? c.tile : a.epi_vec ? c.tile_full : c.tile_scalar);
       t += kper * (n == 1 ? step + c.fill * std::min(1.0, double(blocks) / GEMM_CUS) : double(n) * steps);
       // (the reduce without 8-column runs: 588 x 588 on 6216 pixels 67 us in 2 slices, 55 whole)
-      if (S > 1) t = 1.02 * (t + 4.3 + (0.16e-6 * 4.0 * S + (a.epi_vec ? 0.0 : 4e-6)) * a.M * double(a.N));
+      if (S > 1) t = 1.02 * (t + 3.2 + 0.3 * S + (0.16e-6 * 4.0 * S + (a.epi_vec ? 0.0 : 4e-6)) * a.M * double(a.N));
       if (t < best * 0.999) { best = t; plan = {c.cfg, S}; }
     }
   }
