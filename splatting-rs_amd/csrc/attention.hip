@@ -759,7 +759,7 @@ __global__ void __launch_bounds__(WAVES * 64, QT == 1 ? 4 : 2) attn_bf16_kernel(
 #ifdef SPLAT_ATTN_F32
 // ---------------------------------------------------------------------------------------
 // fp32 path. 4 waves x 32 queries, 32-key tiles. The plain pass (max-free, as in the bf16 kernel)
-// runs S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16: every operand is split exactly
+// runs S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_bf16: every operand is split
 // into three bf16 parts (split8) and the six products down to 2^-18 of the leading one are
 // summed, which keeps fp32's precision at 6/16 of the fp32 instructions' matrix time. Q is split
 // once. The block splits each K and V tile once for its four waves: a thread loads 8 channels of
@@ -771,7 +771,7 @@ __global__ void __launch_bounds__(WAVES * 64, QT == 1 ? 4 : 2) attn_bf16_kernel(
 // The safe pass (running maximum) keeps the operands whole on v_mfma_f32_32x32x2f32, K and V
 // tiles streamed into LDS (rows of 256 bytes, 16-byte chunk c of row r in slot c ^ (r & 15)): k-step j
 // pairs head channels j and j + 32. It also takes the blocks whose plain pass met an infinity, a
-// NaN, or a value that rounds to infinity in bf16.
+// NaN, a value that rounds to infinity in bf16, or one of Q, K or V whose last bits the parts cut.
 template <bool SPLIT>
 __global__ void __launch_bounds__(256, 2) attn_f32_kernel(const AttnArgs p, float c) {
   constexpr int TB = 32 * 256;            // one 32-key fp32 K or V tile (safe pass)

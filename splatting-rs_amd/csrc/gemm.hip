@@ -7,7 +7,7 @@
 // first 16 bytes of a 32-byte k-step, lanes 32-63 the second; A and W use the same k order,
 // so the sum over k is exact whatever order the hardware walks the fragment in.
 //   bf16: one v_mfma_f32_32x32x16_bf16 per k-step;
-//   fp32: 64-byte k-steps (two 16-byte chunks a lane); every float is split exactly into three
+//   fp32: 64-byte k-steps (two 16-byte chunks a lane); every float is split into three
 //   bf16 (split8) and six v_mfma_f32_32x32x16_bf16 sum the products down to 2^-18 of the leading
 //   one (Mfma<float>).
 // Accumulator layout per 32x32 tile (f32x16): lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4,
@@ -1512,6 +1512,7 @@ static bool launch_mfma(const Exec& ex, const GemmArgs& a, int S) {
   const bool tap = a.amode == A_CONV && a.Cin % BK == 0 && a.ks * a.ks <= 32;
   SPLAT_CHECK(a.amode == A_ROWS || tap || !a.relu_in, BAD_ARGUMENT,
               "gemm: ReLU-on-load needs a convolution whose Cin is a multiple of the k-tile");
+  SPLAT_CHECK(a.amode == A_ROWS || sizeof(T) == 2 || a.ks * a.ks <= 32, BAD_ARGUMENT, "gemm: fp32 convolutions of up to 32 taps");
   if (TAP_ONLY) SPLAT_CHECK(tap && epi != EPI_HEAD, BAD_ARGUMENT, "gemm: 32-element k-tiles serve per-tap convs only");
   if (epi == EPI_HEAD) {  // the fused MapAnything head: one tile spans the 128 channels
     SPLAT_CHECK(tap && !a.relu_in && a.N == BN && a.act == ACT_RELU && S == 1, BAD_ARGUMENT, "gemm: fused head");
