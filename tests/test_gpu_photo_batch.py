@@ -126,3 +126,39 @@ def test_one_cpu(ctx):
     finally:
         os.sched_setaffinity(0, cpus)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+def test_two_threads_and_a_busy_stream(ctx):
+    """Two contexts on two threads, each with a ring of its own, behind attention launches still running on
+    their streams."""
+    import threading
+    photos = [_photos(DA3_SIZES), _photos(DA3_SIZES[::-1])]
+    want = [_da3(ctx, p) for p in photos]
+    L, heads = 6000, 6
+    qkv = torch.randn(L, 3 * heads * 64, device="cuda")
+    got, errors = [None, None], []
+
+    def run(k):
+        try:
+            other = splathip.Context(0)
+            W, H = splathip.da3_model_inputs_size([(p.shape[1], p.shape[0]) for p in photos[k]])
+            img = torch.zeros(len(photos[k]), 3, H, W, device="cuda")
+            out = torch.empty(L, heads * 64, device="cuda")
+            torch.cuda.synchronize()
+            for _ in range(3):
+                for _ in range(20):
+                    other.kernel_attention(splathip.F32, qkv.data_ptr(), out.data_ptr(), 1, L, heads)
+                other.da3_model_inputs_device(photos[k], img.data_ptr())
+                other.synchronize()
+                assert np.array_equal(img.cpu().numpy(), want[k][0])
+            got[k] = True
+            other.close()
+        except Exception as e:   # shown by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert not errors and got == [True, True]

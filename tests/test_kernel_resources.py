@@ -56,3 +56,17 @@ def test_fp32_128x128_tiles_fit_twice_a_cu(kernels):
     assert len(tiles) >= 8
     for name, (registers, scratch) in tiles.items():
         assert registers <= 256 and scratch == 0, (name, registers, scratch)
+
+
+def test_fp32_attention_fits_twice_a_cu(kernels):
+    found = {k: v for k, v in kernels.items() if "attn_f32_kernel" in k}
+    assert len(found) == 2
+    for name, (registers, scratch) in found.items():
+        assert registers <= 256 and scratch == 0, (name, registers, scratch)
+
+
+def test_no_fp32_gemm_tile_spills(kernels):
+    """A spilled register is re-read in the k-loop and waits for every load in flight."""
+    tiles = {k: v for k, v in kernels.items() if "gemm_mfma_kernelIf" in k}
+    assert len(tiles) >= 32
+    assert not {k: v for k, v in tiles.items() if v[1] != 0}
